@@ -124,6 +124,38 @@ __device__ __forceinline__ void buf_store(const P& p, rsrc_t r, uint32_t v) {
   using IO = BufIO<sizeof(P), POL>;
   IO::store(__builtin_bit_cast(typename IO::W, p), r, v * static_cast<uint32_t>(sizeof(P)));
 }
+// The same at a byte offset.
+template <class P, int POL = kDefault>
+__device__ __forceinline__ P buf_load_at(rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(P, BufIO<sizeof(P), POL>::load(r, off));
+}
+template <class P, int POL = kDefault>
+__device__ __forceinline__ void buf_store_at(const P& p, rsrc_t r, uint32_t off) {
+  using IO = BufIO<sizeof(P), POL>;
+  IO::store(__builtin_bit_cast(typename IO::W, p), r, off);
+}
+// Where the vectors of a ragged row lie: a row of N >= VEC elements whose width is not a whole number
+// of vectors, or whose base is off the vector's alignment.  Buffer accesses need no alignment
+// (gfx950 runs in unaligned access mode), so vector v of ceil(N / VEC) starts at column
+// min(v VEC, N - VEC): the last one ends with the row and shares `dup` elements with the one
+// before it.  Every access lies inside the row.
+template <class T, int VEC> struct RaggedRow {
+  static constexpr uint32_t kBytes = VEC * sizeof(T);
+  uint32_t nvec, nfull, last, dup;
+  __device__ __forceinline__ explicit RaggedRow(uint32_t N)
+      : nvec((N + VEC - 1) / VEC), nfull(N / VEC),
+        last((N - VEC) * static_cast<uint32_t>(sizeof(T))), dup(nvec * VEC - N) {}
+  // Byte offset of vector v in the row, or one past every resource.
+  __device__ __forceinline__ uint32_t off(uint32_t v) const {
+    const uint32_t o = v * kBytes;
+    return v < nvec ? (o < last ? o : last) : kOutOfRange;
+  }
+  // Elements e >= lo(v) of vector v are its own: those count in sums (lo = VEC: none).
+  __device__ __forceinline__ int lo(uint32_t v) const {
+    return v < nfull ? 0 : v < nvec ? static_cast<int>(dup) : VEC;
+  }
+};
+
 __device__ __forceinline__ void buf_store_f32(float x, rsrc_t r, uint32_t byte_off) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), r, byte_off, 0, 0);
 }

@@ -47,8 +47,25 @@ __device__ __forceinline__ float row_allreduce(float v, float* slot, int wpr, in
 // handled by the hardware range check), so the loop body has no divergent branches.
 // LDS reduction slots are double-buffered by iteration parity: every iteration of a multi-wave
 // row group passes at least one barrier, which separates a slot's reads from its next writes.
-// EXACT: the row is exactly VPL vectors per lane (no masking in the statistics); GELU: 0 none,
-// 1 erf, 2 tanh (a template parameter so the plain kernels carry no GELU code).
+// FIT: kExactFit, the row is exactly VPL vectors per lane (no masking in the statistics);
+// kMaskedFit, whole vectors but masked lanes; kRaggedFit, rows off the 16-byte grid (below).
+// GELU: 0 none, 1 erf, 2 tanh (a template parameter so the plain kernels carry no GELU code).
+//
+// Ragged rows (a width that is not a whole number of 16-byte vectors, or a pointer off a 16-byte
+// boundary) take the same 16-byte accesses, unaligned: gfx950 runs in unaligned access mode, where
+// a buffer load or store needs no alignment.  The row's last vector is moved back to end with the
+// row, so every access lies inside the row and no tail loop is needed; the elements it shares with
+// the vector before it (RaggedRow::lo) are left out of the sums and written twice with the same
+// value.  Column -> lane stays fixed, so gamma and beta stay in registers as on the aligned path.
+// A 16-byte copy at 2-byte alignment moves 5.0-5.4 TB/s here against 5.9 aligned; the scalar path
+// this replaced (one element per lane and load, 128 bytes per wave and instruction) was bound by
+// its load and store issue at 2.2 TB/s.  Forward, us, scalar -> ragged:
+//   LayerNorm bf16 8192 x 4098 50.6 -> 28.2, 8192 x 4095 35.3 -> 27.0, 4000 x 4097 28.8 -> 18.9,
+//   4000 x 9999 55.1 -> 35.2, 16384 x 1023 18.2 -> 14.9; fp32 5000 x 5003 43.4 -> 39.9; residual +
+//   LayerNorm bf16 8000 x 2050 43.9 -> 26.2; LN + GELU erf bf16 14591 x 1146 34.9 -> 22.5, tanh
+//   fp16 6001 x 1023 12.0 -> 10.0; LN -> fp8 bf16 9000 x 3001 41.3 -> 23.7; LN -> MXFP8 bf16 4096
+//   x 4096 off alignment 29.5 -> 14.3.  What bounds it now: the unaligned rate for many rows, ramp
+//   and drain for few.
 // ---------------------------------------------------------------------------------------------
 // Rows in flight ahead of the current one: about 64 bytes of loads per lane.  A lane holding 64
 // bytes or more of a row prefetches one row, a smaller slice two (measured with exact ring
@@ -89,9 +106,7 @@ __device__ __forceinline__ float row_allreduce(float v, float* slot, int wpr, in
 template <class T, int FP8, bool RES, int GELU, int VEC, int VPL, int MAXT>
 constexpr int fwd_prefetch_depth() {
   constexpr bool raw = MAXT > 256 && VPL * VEC >= 32;
-  constexpr bool params_in_lds =
-      MAXT == 1024 && ((raw && VEC > 1 && sizeof(T) == 2) || (VEC == 1 && VPL == 16 &&
-                                                               sizeof(T) <= 4));
+  constexpr bool params_in_lds = MAXT == 1024 && raw && sizeof(T) == 2;
   constexpr bool odd_two =
       VEC == 8 && MAXT == 256 && !RES && GELU == 0 && FP8 == 0 && (VPL == 5 || VPL == 7);
   return (params_in_lds && raw && !RES) || odd_two
@@ -99,18 +114,21 @@ constexpr int fwd_prefetch_depth() {
              : FLN_FWD_PREFETCH(VPL * VEC * static_cast<int>(sizeof(T)), MAXT);
 }
 
-template <class T, int FP8, bool RES, int GELU, int VEC, int VPL, bool EXACT, int MAXT>
+constexpr int kMaskedFit = 0, kExactFit = 1, kRaggedFit = 2;
+
+template <class T, int FP8, bool RES, int GELU, int VEC, int VPL, int FIT, int MAXT>
 __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_t row_blocks) {
+  constexpr bool EXACT = FIT == kExactFit;
+  constexpr bool RAGGED = FIT == kRaggedFit;
   constexpr bool RAW = MAXT > 256 && VPL * VEC >= 32;  // row kept in the I/O type
+  static_assert(!(RAGGED && RAW), "ragged rows: no raw tiles");
   // gamma / beta parked in LDS, each thread its own copy (no barrier; 64-128 KiB), for the 16-bit
-  // RAW tiles and the scalar path's 16 elements per lane in 1024-thread blocks: in registers
+  // RAW tiles: in registers
   // they made the residual / fp8 flavours spill 16-332 B per lane, and they left room for only
   // one row in flight elsewhere (bf16, us: residual + LN 2048 x 32768 102.7 -> 89.6, residual +
   // RMSNorm -> fp8 111.9 -> 82.3; with two rows in flight LN 2048 x 32768 52.8 -> 48.8, RMSNorm
   // 4096 x 20480 62.6 -> 57.9, LN -> fp8 4096 x 20480 73.5 -> 67.1).
-  constexpr bool PARAMS_IN_LDS =
-      MAXT == 1024 && ((RAW && VEC > 1 && sizeof(T) == 2) || (VEC == 1 && VPL == 16 &&
-                                                                sizeof(T) <= 4));
+  constexpr bool PARAMS_IN_LDS = MAXT == 1024 && RAW && sizeof(T) == 2;
   // rows in flight ahead of the current one (the residual flavour's second input leaves room for
   // one only)
   constexpr int PD = fwd_prefetch_depth<T, FP8, RES, GELU, VEC, VPL, MAXT>();
@@ -128,8 +146,21 @@ __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_
   const int tpr = kWave * wpr;
   const int rows_per_block = blockDim.x / tpr;
   const int64_t N = p.cols;
-  const int nvec = static_cast<int>(N / VEC);
+  const int nvec = static_cast<int>(N / VEC);  // whole vectors
   const uint32_t row_bytes = static_cast<uint32_t>(N * sizeof(T));
+  // Byte offset of this lane's vector slot i in a row.
+  const RaggedRow<T, VEC> rag(static_cast<uint32_t>(RAGGED ? N : VEC));
+  uint32_t rag_off[RAGGED ? VPL : 1];
+  if constexpr (RAGGED) {
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) rag_off[i] = rag.off(static_cast<uint32_t>(t + i * tpr));
+  }
+  auto off = [&](int i) -> uint32_t {
+    if constexpr (RAGGED)
+      return rag_off[i];
+    else
+      return static_cast<uint32_t>(t + i * tpr) * static_cast<uint32_t>(sizeof(P));
+  };
   // mean = sum / N as sum * (1/N) plus one FMA correction step, which returns the exact quotient
   // whenever it is representable (an exactly summed constant row then maps to beta exactly)
   // without the long correctly-rounded division sequence.
@@ -147,19 +178,19 @@ __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_
   if constexpr (PARAMS_IN_LDS) {
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      P g0 = buf_load<P>(g_rs, t + i * tpr);
+      P g0 = buf_load_at<P>(g_rs, off(i));
       if (p.gamma == nullptr) {  // absent gamma multiplies by one (uniform)
 #pragma unroll
         for (int e = 0; e < VEC; ++e) g0.v[e] = static_cast<T>(1.0f);
       }
       gsh[i * MAXT + threadIdx.x] = g0;
-      bsh[i * MAXT + threadIdx.x] = buf_load<P>(b_rs, t + i * tpr);
+      bsh[i * MAXT + threadIdx.x] = buf_load_at<P>(b_rs, off(i));
     }
   } else {
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {  // unconditional: an absent tensor has a zero-byte resource
-      gv[i] = buf_load<P>(g_rs, t + i * tpr);
-      bv[i] = buf_load<P>(b_rs, t + i * tpr);  // absent beta reads as zeros: adds nothing
+      gv[i] = buf_load_at<P>(g_rs, off(i));
+      bv[i] = buf_load_at<P>(b_rs, off(i));  // absent beta reads as zeros: adds nothing
     }
     if (p.gamma == nullptr) {  // absent gamma multiplies by one (uniform, once per kernel)
 #pragma unroll
@@ -169,17 +200,41 @@ __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_
     }
   }
   // Vector slot i is complete (no lane past the row) when (i + 1) * tpr <= nvec; only the
-  // other slots need per-element masks in the centred sums and the fp8 row max.
+  // other slots need per-element masks in the centred sums and the fp8 row max (ragged rows: in
+  // the plain sum as well, for the elements that the last vector shares with the one before).
   auto slot_full = [&](int i) { return EXACT || (i + 1) * tpr <= nvec; };
+  // Ragged rows: one slot at most is partly filled; the slots after it are empty (skipped).  lo:
+  // this lane's first element of that slot that counts in sums (VEC: none), made opaque per row:
+  // hoisted, its VEC compare masks would live in (and spill from) SGPR pairs.
+  int tail_slot = 0;  // (nvec - 1) / tpr
+  if constexpr (RAGGED) {
+#pragma unroll
+    for (int i = 1; i < VPL; ++i) tail_slot += static_cast<uint32_t>(i * tpr) < rag.nvec ? 1 : 0;
+  }
+  const int tail_lo = RAGGED ? rag.lo(static_cast<uint32_t>(t + tail_slot * tpr)) : 0;
+  auto slot_lo = [&](int i) -> int {
+    if constexpr (RAGGED) {
+      int lo = tail_lo;
+      asm volatile("" : "+v"(lo));
+      return lo;
+    } else {
+      return (t + i * tpr) < nvec ? 0 : VEC;
+    }
+  };
   // Elements of the row held by wave w of a row group (w < wpr), and this wave's reciprocal.
   auto wave_elems = [&](int w) -> float {
     int n = 0;
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      const int left = nvec - (i * tpr + w * kWave);
-      n += left <= 0 ? 0 : (left < kWave ? left : kWave);
+      if constexpr (RAGGED) {
+        const int left = static_cast<int>(N) - (i * tpr + w * kWave) * VEC;
+        n += left <= 0 ? 0 : (left < kWave * VEC ? left : kWave * VEC);
+      } else {
+        const int left = nvec - (i * tpr + w * kWave);
+        n += VEC * (left <= 0 ? 0 : (left < kWave ? left : kWave));
+      }
     }
-    return static_cast<float>(n * VEC);
+    return static_cast<float>(n);
   };
   const float own_n = wave_elems(wave - rg * wpr);
   const float inv_wave_n = own_n > 0.0f ? 1.0f / own_n : 0.0f;
@@ -196,11 +251,11 @@ __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_
     const uint32_t nb = bytes_of(rb);
     const rsrc_t xr = make_rsrc(X + row * N, nb);
 #pragma unroll
-    for (int i = 0; i < VPL; ++i) xv[slot][i] = buf_load<P, FLN_FWD_LOAD_POL>(xr, t + i * tpr);
+    for (int i = 0; i < VPL; ++i) xv[slot][i] = buf_load_at<P, FLN_FWD_LOAD_POL>(xr, off(i));
     if constexpr (RES) {
       const rsrc_t rr = make_rsrc(R + row * N, nb);
 #pragma unroll
-      for (int i = 0; i < VPL; ++i) rv[slot][i] = buf_load<P, FLN_FWD_LOAD_POL>(rr, t + i * tpr);
+      for (int i = 0; i < VPL; ++i) rv[slot][i] = buf_load_at<P, FLN_FWD_LOAD_POL>(rr, off(i));
     }
   };
 
@@ -294,12 +349,12 @@ __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_
             const float d = xin(i, e) - c;
             acc = fmaf(d, d, acc);
           }
-        } else {
-          const bool ok = (t + i * tpr) < nvec;
+        } else if (!RAGGED || i == tail_slot) {
+          const int lo = slot_lo(i);
 #pragma unroll
           for (int e = 0; e < VEC; ++e) {
             const float d = xin(i, e) - c;
-            acc += ok ? d * d : 0.0f;
+            acc += e >= lo ? d * d : 0.0f;
           }
         }
       }
@@ -311,9 +366,16 @@ __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_
     } else {
       float s = 0.0f;
 #pragma unroll
-      for (int i = 0; i < VPL; ++i)
+      for (int i = 0; i < VPL; ++i) {
+        if (!RAGGED || slot_full(i)) {
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) s += xin(i, e);
+          for (int e = 0; e < VEC; ++e) s += xin(i, e);
+        } else if (i == tail_slot) {
+          const int lo = slot_lo(i);
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) s += e >= lo ? xin(i, e) : 0.0f;
+        }
+      }
       const float sw = wave_allreduce<SumOp>(s);
       if (wpr == 1) {
         mean = sw * inv_n;
@@ -416,8 +478,8 @@ __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_
         if (slot_full(i)) {
 #pragma unroll
           for (int e = 0; e < VEC; ++e) am = fmaxf(am, fabsf(out(i, e)));
-        } else {
-          const bool ok = (t + i * tpr) < nvec;
+        } else if (!RAGGED || i == tail_slot) {
+          const bool ok = slot_lo(i) < VEC;
 #pragma unroll
           for (int e = 0; e < VEC; ++e) am = fmaxf(am, ok ? fabsf(out(i, e)) : 0.0f);
         }
@@ -456,12 +518,12 @@ __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_
     if constexpr (RES) {
       const rsrc_t hr = make_rsrc(p.h ? static_cast<T*>(p.h) + row * N : nullptr, nb);
 #pragma unroll
-      for (int i = 0; i < VPL; ++i) buf_store<P, FLN_FWD_STORE_POL>(ho[i], hr, t + i * tpr);
+      for (int i = 0; i < VPL; ++i) buf_store_at<P, FLN_FWD_STORE_POL>(ho[i], hr, off(i));
     }
     if constexpr (FP8 == 0) {
       const rsrc_t yr = make_rsrc(static_cast<T*>(p.y) + row * N, nb);
 #pragma unroll
-      for (int i = 0; i < VPL; ++i) buf_store<P, FLN_FWD_STORE_POL>(yo[i], yr, t + i * tpr);
+      for (int i = 0; i < VPL; ++i) buf_store_at<P, FLN_FWD_STORE_POL>(yo[i], yr, off(i));
     } else {
       if constexpr (FP8 == 2) {
         // One E8M0 byte per block, stored by the block's first lane.
@@ -482,8 +544,10 @@ __global__ __launch_bounds__(MAXT) void fwd_reg_kernel(const FwdParams p, int64_
 #pragma unroll
       for (int i = 0; i < VPL; ++i) {
         if constexpr (VEC >= 4)
-          BufIO<VEC, FLN_FWD_STORE_POL>::store(qo[i], qr,
-                                               (t + i * tpr) * static_cast<uint32_t>(VEC));
+          BufIO<VEC, FLN_FWD_STORE_POL>::store(
+              qo[i], qr,  // ragged: an offset out of range stays so
+              RAGGED ? off(i) / static_cast<uint32_t>(sizeof(T))
+                     : (t + i * tpr) * static_cast<uint32_t>(VEC));
         else
           __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(qo[i]), qr, t + i * tpr,
                                                0, FLN_FWD_STORE_POL);
@@ -751,10 +815,9 @@ __global__ __launch_bounds__(kFwdLdsThreads) void fwd_lds_kernel(const FwdParams
 
 // ---------------------------------------------------------------------------------------------
 // Rows past the LDS tile (16-bit rows of more than 65536 columns, fp32 rows of more than 32768)
-// and long rows off the vector path: one 1024-thread block per row at a time, rows
+// and long ragged rows (more than 16384 columns): one 1024-thread block per row at a time, rows
 // grid-stride, each pass streaming the row in steps of U vectors per thread (64 bytes: 4
-// vectors, or 16-32 elements on the scalar path; thread t reads vectors base + t + 1024 u, so
-// every wave-wide access is coalesced):
+// vectors; thread t reads vectors base + t + 1024 u, so every wave-wide access is coalesced):
 //   pass 1, statistics: per thread, each step's valid elements are reduced to (count, mean,
 //     centred sum of squares) and merged into the thread's running triple (the pairwise update
 //     of Chan, Golub and LeVeque); the block's mean is then the sum of count x mean over the
@@ -771,7 +834,7 @@ __global__ __launch_bounds__(kFwdLdsThreads) void fwd_lds_kernel(const FwdParams
 constexpr int kFwdWideThreads = 1024;
 constexpr int kFwdWideStepBytes = 64;  // bytes of the row per thread and step (4 vectors)
 
-template <class T, int FP8, bool RES, int GELU, int VEC>
+template <class T, int FP8, bool RES, int GELU, int VEC, bool RAGGED>
 __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdParams p) {
   constexpr int kT = kFwdWideThreads;
   constexpr int kW = kT / kWave;
@@ -792,7 +855,11 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
   const int lane = t & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int64_t N = p.cols;
-  const uint32_t nvec = static_cast<uint32_t>(N / VEC);
+  const RaggedRow<T, VEC> rag(static_cast<uint32_t>(RAGGED ? N : VEC));
+  const uint32_t nvec = RAGGED ? rag.nvec : static_cast<uint32_t>(N / VEC);
+  auto off = [&](uint32_t v) -> uint32_t {  // byte offset of vector v in a row
+    return RAGGED ? rag.off(v) : v * static_cast<uint32_t>(sizeof(P));
+  };
   const uint32_t row_bytes = static_cast<uint32_t>(N * sizeof(T));
   const float fn = static_cast<float>(N);
   const float inv_n = 1.0f / fn;
@@ -814,8 +881,9 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
       P rv[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        hv[u] = buf_load<P, POL>(xq, base + t + kT * u);
-        if constexpr (RES) rv[u] = buf_load<P, POL>(rq, base + t + kT * u);
+        const uint32_t o = off(base + t + kT * u);
+        hv[u] = buf_load_at<P, POL>(xq, o);
+        if constexpr (RES) rv[u] = buf_load_at<P, POL>(rq, o);
       }
       if constexpr (RES) {
 #pragma unroll
@@ -836,21 +904,34 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
     for (uint32_t base = 0; base < nvec; base += kT * U) {
       P hv[U];
       load_step(base, hv, Keep{});
+      // A ragged row's last step: its last vector counts only its own elements.
+      const bool tail = RAGGED && base + kT * U > rag.nfull;  // uniform
       if constexpr (RES) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) buf_store<P, FLN_FWD_STORE_POL>(hv[u], hr, base + t + kT * u);
+        for (int u = 0; u < U; ++u)
+          buf_store_at<P, FLN_FWD_STORE_POL>(hv[u], hr, off(base + t + kT * u));
       }
       if (p.rms) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+          const int lo = tail ? rag.lo(base + t + kT * u) : 0;
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) m2 = fmaf(to_f32(hv[u].v[e]), to_f32(hv[u].v[e]), m2);
+          for (int e = 0; e < VEC; ++e) {
+            const float d = tail && e < lo ? 0.0f : to_f32(hv[u].v[e]);
+            m2 = fmaf(d, d, m2);
+          }
+        }
         continue;
       }
       float c = 0.0f, s = 0.0f;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        if (base + t + kT * u < nvec) {
+        if (tail) {
+          const int lo = rag.lo(base + t + kT * u);
+          c += static_cast<float>(VEC - lo);
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) s += e >= lo ? to_f32(hv[u].v[e]) : 0.0f;
+        } else if (base + t + kT * u < nvec) {
           c += static_cast<float>(VEC);
 #pragma unroll
           for (int e = 0; e < VEC; ++e) s += to_f32(hv[u].v[e]);
@@ -861,7 +942,14 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
         float q = 0.0f;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          if (base + t + kT * u < nvec) {
+          if (tail) {
+            const int lo = rag.lo(base + t + kT * u);
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+              const float d = to_f32(hv[u].v[e]) - mg;
+              q += e >= lo ? d * d : 0.0f;
+            }
+          } else if (base + t + kT * u < nvec) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
               const float d = to_f32(hv[u].v[e]) - mg;
@@ -911,8 +999,8 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const uint32_t v = base + t + kT * u;
-          const P gv = buf_load<P>(g_rs, v);
-          const P bv = buf_load<P>(b_rs, v);
+          const P gv = buf_load_at<P>(g_rs, off(v));
+          const P bv = buf_load_at<P>(b_rs, off(v));
           if (v < nvec) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) am = fmaxf(am, fabsf(affine(hv[u], gv, bv, e)));
@@ -932,8 +1020,8 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const uint32_t v = base + t + kT * u;
-        const P gv = buf_load<P>(g_rs, v);
-        const P bv = buf_load<P>(b_rs, v);
+        const P gv = buf_load_at<P>(g_rs, off(v));
+        const P bv = buf_load_at<P>(b_rs, off(v));
         float a[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) a[e] = affine(hv[u], gv, bv, e);
@@ -941,8 +1029,8 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
           P o;
 #pragma unroll
           for (int e = 0; e < VEC; ++e) o.v[e] = from_f32<T>(a[e]);
-          buf_store<P, FLN_FWD_STORE_POL>(o, make_rsrc(static_cast<T*>(p.y) + row * N, row_bytes),
-                                          v);
+          buf_store_at<P, FLN_FWD_STORE_POL>(
+              o, make_rsrc(static_cast<T*>(p.y) + row * N, row_bytes), off(v));
         } else {
           float m = inv;
           if constexpr (FP8 == 2) {
@@ -960,19 +1048,19 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
                                                  v % G == 0 ? v / G : kOutOfRange, 0, 0);
           }
           // Per-row scale: |a * inv| <= 448 (1 + 2^-22) < 464, but the saturating form is kept
-          // (the scalar path converts one element at a time).
+          // (this kernel is not bound by its VALU work).
+          const uint32_t qo = RAGGED ? off(v) / static_cast<uint32_t>(sizeof(T))
+                                     : v * static_cast<uint32_t>(VEC);  // one byte an element
           const rsrc_t qr = make_rsrc(static_cast<uint8_t*>(p.y) + row * N,
                                       static_cast<uint32_t>(N));
           if constexpr (VEC == 8) {
             u32x2 w;
             w.x = fp8x4(a[0] * m, a[1] * m, a[2] * m, a[3] * m);
             w.y = fp8x4(a[4] * m, a[5] * m, a[6] * m, a[7] * m);
-            BufIO<8, FLN_FWD_STORE_POL>::store(w, qr, v * 8u);
-          } else if constexpr (VEC == 4) {
-            BufIO<4, FLN_FWD_STORE_POL>::store(fp8x4(a[0] * m, a[1] * m, a[2] * m, a[3] * m), qr,
-                                               v * 4u);
+            BufIO<8, FLN_FWD_STORE_POL>::store(w, qr, qo);
           } else {
-            __builtin_amdgcn_raw_buffer_store_b8(fp8x1(a[0] * m), qr, v, 0, FLN_FWD_STORE_POL);
+            BufIO<4, FLN_FWD_STORE_POL>::store(fp8x4(a[0] * m, a[1] * m, a[2] * m, a[3] * m), qr,
+                                               qo);
           }
         }
       }
@@ -1117,7 +1205,7 @@ int64_t resident_blocks(K kernel, int threads, std::atomic<int>* cache_per_devic
   return static_cast<int64_t>(per_cu) * device_cu_count();
 }
 
-template <class T, int FP8, bool RES, int GELU, int VEC, int VPL, bool EXACT, int MAXT>
+template <class T, int FP8, bool RES, int GELU, int VEC, int VPL, int FIT, int MAXT>
 int launch_reg_t(const FwdParams& p, int threads, hipStream_t s) {
   // The exact-GELU kernels fill their LDS table with one entry per thread.
   if (GELU == 1 && threads < kGeluLogTabN) return FLN_ERR_INVALID;
@@ -1125,7 +1213,7 @@ int launch_reg_t(const FwdParams& p, int threads, hipStream_t s) {
     return FLN_ERR_INVALID;
   const int rows_per_block = threads / (kWave * p.wpr);
   const int64_t row_blocks = (p.rows + rows_per_block - 1) / rows_per_block;
-  auto kernel = fwd_reg_kernel<T, FP8, RES, GELU, VEC, VPL, EXACT, MAXT>;
+  auto kernel = fwd_reg_kernel<T, FP8, RES, GELU, VEC, VPL, FIT, MAXT>;
   // Per instantiation, [waves per block][device]: one instantiation runs with several block
   // sizes (a 1024-thread one with 5-16 waves per row, one row per block).
   static std::atomic<int> occupancy_cache[MAXT / kWave + 1][64];
@@ -1163,76 +1251,89 @@ int launch_reg_t(const FwdParams& p, int threads, hipStream_t s) {
   return launch_cached(kernel, fn_cache, dim3(grid), dim3(threads), s, p, row_blocks);
 }
 
-template <class T, int FP8, bool RES, int GELU, int VEC, int VPL, bool EXACT>
+template <class T, int FP8, bool RES, int GELU, int VEC, int VPL, int FIT>
 int launch_reg(const FwdParams& p, int threads, hipStream_t s) {
-  if (threads <= 256) return launch_reg_t<T, FP8, RES, GELU, VEC, VPL, EXACT, 256>(p, threads, s);
-  return launch_reg_t<T, FP8, RES, GELU, VEC, VPL, EXACT, 1024>(p, threads, s);
+  if (threads <= 256) return launch_reg_t<T, FP8, RES, GELU, VEC, VPL, FIT, 256>(p, threads, s);
+  // Scalar rows are one or two waves each; ragged ones have no raw tiles.
+  if constexpr (VEC > 1 && (FIT != kRaggedFit || VPL * VEC < 32))
+    return launch_reg_t<T, FP8, RES, GELU, VEC, VPL, FIT, 1024>(p, threads, s);
+  return FLN_ERR_INVALID;
 }
 
 // Largest vectors-per-lane instantiated: 32 elements per lane for 16-byte vectors (keeps a
-// LayerNorm row slice, its fp32 copy and the affine parameters within ~120 VGPRs), 16 for the
-// scalar path.
-template <int VEC> constexpr int max_vpl() { return VEC == 1 ? 16 : 32 / VEC; }
+// LayerNorm row slice, its fp32 copy and the affine parameters within ~120 VGPRs); 4 elements
+// on the scalar path (rows of at most kScalarCols columns, one or two waves each).
+constexpr int64_t kScalarCols = 256;
+template <int VEC> constexpr int max_vpl() { return VEC == 1 ? kScalarCols / kWave : 32 / VEC; }
 
 template <class T, int FP8, bool RES, int GELU, int VEC, int VPL>
-int launch_reg_exact(const FwdParams& p, bool exact, int threads, hipStream_t s) {
-  // The exact (mask-free) variant is only instantiated for 16-byte vectors.
-  if constexpr (VEC > 1)
-    if (exact) return launch_reg<T, FP8, RES, GELU, VEC, VPL, true>(p, threads, s);
-  return launch_reg<T, FP8, RES, GELU, VEC, VPL, false>(p, threads, s);
+int launch_reg_fit(const FwdParams& p, int fit, int threads, hipStream_t s) {
+  // The exact (mask-free) and ragged variants are only instantiated for 16-byte vectors.
+  if constexpr (VEC > 1) {
+    if (fit == kExactFit)
+      return launch_reg<T, FP8, RES, GELU, VEC, VPL, kExactFit>(p, threads, s);
+    if constexpr (VPL * VEC < 32 || VEC == 8)
+      if (fit == kRaggedFit)
+        return launch_reg<T, FP8, RES, GELU, VEC, VPL, kRaggedFit>(p, threads, s);
+    if (fit == kRaggedFit) return FLN_ERR_INVALID;  // no ragged tile of 8 fp32 vectors
+  }
+  return launch_reg<T, FP8, RES, GELU, VEC, VPL, kMaskedFit>(p, threads, s);
 }
 
 template <class T, int FP8, bool RES, int GELU, int VEC, int VPL>
-int launch_reg_odd(const FwdParams& p, bool exact, int threads, hipStream_t s) {
+int launch_reg_odd(const FwdParams& p, int fit, int threads, hipStream_t s) {
   // The flavours the plan gives these tiles: GELU only as LN + GELU; with a residual 3 or 5
   // vectors per lane (6 and 7 need AGPRs there); MX outputs only with a residual; 6 vectors for
   // the fp8 row scale and GELU.
   constexpr bool kPlanned =
       VEC == 8 && (GELU == 0 || (FP8 == 0 && !RES)) && (!RES || VPL == 3 || VPL == 5) &&
       (FP8 != 2 || RES) && (VPL != 6 || (FP8 == 1 && !RES) || GELU != 0);
+  // Ragged rows: 3 and 5 vectors per lane in every flavour.
+  if constexpr (VEC == 8 && (VPL == 3 || VPL == 5))
+    if (fit == kRaggedFit && threads <= 256)
+      return launch_reg_t<T, FP8, RES, GELU, VEC, VPL, kRaggedFit, 256>(p, threads, s);
   if constexpr (kPlanned)
-    if (exact && threads <= 256)
-      return launch_reg_t<T, FP8, RES, GELU, VEC, VPL, true, 256>(p, threads, s);
+    if (fit == kExactFit && threads <= 256)
+      return launch_reg_t<T, FP8, RES, GELU, VEC, VPL, kExactFit, 256>(p, threads, s);
   return FLN_ERR_INVALID;
 }
 
 template <class T, int FP8, bool RES, int GELU, int VEC>
-int launch_reg_vpl(const FwdParams& p, int vpl, bool exact, int threads, hipStream_t s) {
+int launch_reg_vpl(const FwdParams& p, int vpl, int fit, int threads, hipStream_t s) {
   constexpr int CAP = max_vpl<VEC>();
-  switch (vpl) {
-    case 1: return launch_reg_exact<T, FP8, RES, GELU, VEC, 1>(p, exact, threads, s);
-    case 2: return launch_reg_exact<T, FP8, RES, GELU, VEC, 2>(p, exact, threads, s);
-    case 4: return launch_reg_exact<T, FP8, RES, GELU, VEC, 4>(p, exact, threads, s);
-    // Odd and six-vector tiles (3, 5, 6, 7 vectors per lane): exact tilings only, in blocks of at
-    // most 256 threads, for the 16-bit flavours that the plan gives them.
-    case 3: return launch_reg_odd<T, FP8, RES, GELU, VEC, 3>(p, exact, threads, s);
-    case 5: return launch_reg_odd<T, FP8, RES, GELU, VEC, 5>(p, exact, threads, s);
-    case 6: return launch_reg_odd<T, FP8, RES, GELU, VEC, 6>(p, exact, threads, s);
-    case 7: return launch_reg_odd<T, FP8, RES, GELU, VEC, 7>(p, exact, threads, s);
-    case 8:
-      if constexpr (CAP >= 8)
-        return launch_reg_exact<T, FP8, RES, GELU, VEC, 8>(p, exact, threads, s);
-      return FLN_ERR_INVALID;
-    case 16:
-      if constexpr (CAP >= 16)
-        return launch_reg_exact<T, FP8, RES, GELU, VEC, 16>(p, exact, threads, s);
-      return FLN_ERR_INVALID;
-    default: return FLN_ERR_INVALID;
+  if constexpr (CAP > 1) {
+    switch (vpl) {
+      case 2: return launch_reg_fit<T, FP8, RES, GELU, VEC, 2>(p, fit, threads, s);
+      case 4: return launch_reg_fit<T, FP8, RES, GELU, VEC, 4>(p, fit, threads, s);
+      // Odd and six-vector tiles (3, 5, 6, 7 vectors per lane): exact tilings only, in blocks of
+      // at most 256 threads, for the 16-bit flavours that the plan gives them.
+      case 3: return launch_reg_odd<T, FP8, RES, GELU, VEC, 3>(p, fit, threads, s);
+      case 5: return launch_reg_odd<T, FP8, RES, GELU, VEC, 5>(p, fit, threads, s);
+      case 6: return launch_reg_odd<T, FP8, RES, GELU, VEC, 6>(p, fit, threads, s);
+      case 7: return launch_reg_odd<T, FP8, RES, GELU, VEC, 7>(p, fit, threads, s);
+      case 8:
+        if constexpr (CAP >= 8)
+          return launch_reg_fit<T, FP8, RES, GELU, VEC, 8>(p, fit, threads, s);
+        return FLN_ERR_INVALID;
+      default: break;
+    }
   }
+  if (vpl == 1) return launch_reg_fit<T, FP8, RES, GELU, VEC, 1>(p, fit, threads, s);
+  return FLN_ERR_INVALID;
 }
 
 // Flavour dispatch: GELU only exists without residual and fp8 output.  FP8: 0 none, 1 fp8 with
 // a per-row scale, 2 OCP MX fp8 (E8M0 scale per 32 elements).
 template <class T, int FP8, int VEC>
-int launch_reg_flavour(const FwdParams& p, int vpl, bool exact, int threads, hipStream_t s) {
-  if (p.res) return launch_reg_vpl<T, FP8, true, 0, VEC>(p, vpl, exact, threads, s);
+int launch_reg_flavour(const FwdParams& p, int vpl, int fit, int threads, hipStream_t s) {
+  if (p.res) return launch_reg_vpl<T, FP8, true, 0, VEC>(p, vpl, fit, threads, s);
   if constexpr (FP8 == 0) {
     if (p.gelu == FLN_GELU_ERF)
-      return launch_reg_vpl<T, false, false, 1, VEC>(p, vpl, exact, threads, s);
+      return launch_reg_vpl<T, false, false, 1, VEC>(p, vpl, fit, threads, s);
     if (p.gelu == FLN_GELU_TANH)
-      return launch_reg_vpl<T, false, false, 2, VEC>(p, vpl, exact, threads, s);
+      return launch_reg_vpl<T, false, false, 2, VEC>(p, vpl, fit, threads, s);
   }
-  return launch_reg_vpl<T, FP8, false, 0, VEC>(p, vpl, exact, threads, s);
+  return launch_reg_vpl<T, FP8, false, 0, VEC>(p, vpl, fit, threads, s);
 }
 
 template <class T, int FP8, int VEC>
@@ -1691,7 +1792,7 @@ inline bool overlaps(const void* a, int64_t na, const void* b, int64_t nb) {
   return x < y + static_cast<uintptr_t>(nb) && y < x + static_cast<uintptr_t>(na);
 }
 
-template <class T, int FP8, int VEC>
+template <class T, int FP8, int VEC, bool RAGGED>
 int launch_wide(const FwdParams& p, hipStream_t s) {
   auto launch = [&](auto kernel) {
     static std::atomic<int> occupancy_cache[64];  // per instantiation, per device
@@ -1703,12 +1804,12 @@ int launch_wide(const FwdParams& p, hipStream_t s) {
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kFwdWideThreads), 0, s, p);
     return static_cast<int>(hipGetLastError());
   };
-  if (p.res) return launch(fwd_wide_kernel<T, FP8, true, 0, VEC>);
+  if (p.res) return launch(fwd_wide_kernel<T, FP8, true, 0, VEC, RAGGED>);
   if constexpr (FP8 == 0) {
-    if (p.gelu == FLN_GELU_ERF) return launch(fwd_wide_kernel<T, 0, false, 1, VEC>);
-    if (p.gelu == FLN_GELU_TANH) return launch(fwd_wide_kernel<T, 0, false, 2, VEC>);
+    if (p.gelu == FLN_GELU_ERF) return launch(fwd_wide_kernel<T, 0, false, 1, VEC, RAGGED>);
+    if (p.gelu == FLN_GELU_TANH) return launch(fwd_wide_kernel<T, 0, false, 2, VEC, RAGGED>);
   }
-  return launch(fwd_wide_kernel<T, FP8, false, 0, VEC>);
+  return launch(fwd_wide_kernel<T, FP8, false, 0, VEC, RAGGED>);
 }
 
 template <class T, class A, int FP8>
@@ -1799,6 +1900,49 @@ inline FwdGeometry fwd_geometry(int64_t rows, int64_t nvec, int cap, int wide_ca
   return g;
 }
 
+// The tiling of ragged rows, whose width is as a rule no whole tile: the fewest waves per row whose
+// tile holds at most 1/8 more vectors than the tightest one.  Masked slots cost issue slots, and
+// extra waves cross-wave reductions (LayerNorm, us, waves x vectors per lane): bf16 4000 x 4097
+// (513 vectors) 2 x 5 15.9, 3 x 3 16.6, 9 x 1 17.4, 4 x 4 20.3; 6000 x 6001 3 x 4 31.8, 12 x 1
+// 31.5, 2 x 8 does not fit; 4000 x 9999 10 x 2 35.1, 4 x 5 37.8, 16 x 2 42.2; fp32 3000 x 3003
+// 3 x 4 15.6, 2 x 8 16.8; 5000 x 5003 5 x 4 38.2, 4 x 8 41.4; residual + LayerNorm bf16 8000 x
+// 2050 1 x 5 26.0, 2 x 4 28.5.  Vectors per lane: of 16-bit rows up to 4 in one to four waves (5 in
+// one or two) and up to 2 in more; of fp32 rows 1, 2 or 4 (16 waves x 4: 16384 columns, the 16-bit
+// limit 16 x 2).  Longer rows take the streamed kernel.
+inline FwdGeometry ragged_geometry(int64_t rows, int64_t nvec, int vec, bool erf, int forced_wpr,
+                                   int64_t cus) {
+  FwdGeometry g{};
+  constexpr int max_wpr = 16;
+  auto tile = [&](int w) -> int {  // vectors per lane over w waves, 0 where there is no such tile
+    const int64_t v = (nvec + kWave * w - 1) / (kWave * w);
+    if (vec == 4) return v > 4 ? 0 : v == 3 ? 4 : static_cast<int>(v);
+    if (w > 4) return v > 2 ? 0 : static_cast<int>(v);
+    if (erf && w == 3 && v > 2) return 0;  // the exact GELU's table wants whole 256-thread blocks
+    return v > 5 || (v == 5 && w > 2) ? 0 : static_cast<int>(v);
+  };
+  int64_t tightest = 0;
+  for (int w = 1; w <= max_wpr; ++w) {
+    const int64_t slots = static_cast<int64_t>(tile(w)) * w;
+    if (slots > 0 && (tightest == 0 || slots < tightest)) tightest = slots;
+  }
+  if (tightest == 0) {
+    g.loop = true;
+    return g;
+  }
+  int wpr = 1;
+  while (tile(wpr) == 0 || static_cast<int64_t>(tile(wpr)) * wpr * 8 > tightest * 9) ++wpr;
+  // Few rows: more waves per row, up to 4, as for aligned rows, while that leaves each lane fewer
+  // vectors (exact GELU, fp32 17 x 1023, 256 vectors: 4 x 1 4.5, 2 x 2 5.3).
+  while (rows * wpr < 4 * cus && wpr * 2 <= 4 && tile(wpr * 2) > 0 &&
+         tile(wpr * 2) < tile(wpr))
+    wpr *= 2;
+  if (forced_wpr >= 1 && forced_wpr <= max_wpr && tile(forced_wpr) > 0) wpr = forced_wpr;
+  g.wpr = wpr;
+  g.vpl = tile(wpr);
+  g.threads = (4 % wpr == 0) ? 256 : kWave * wpr;
+  return g;
+}
+
 // The launch plan of a forward call: which kernel route runs and its tiling.  The dispatcher
 // below and the C-ABI query fln_forward_plan (what functional.get_optimal_config reports) both
 // take it from here, so there is one rule.  Inputs besides the shape: the flavour (fp8 / MX
@@ -1807,7 +1951,7 @@ inline FwdGeometry fwd_geometry(int64_t rows, int64_t nvec, int cap, int wide_ca
 // for fp8 codes, is 16-byte aligned), and the CU count.
 struct FwdPlan {
   int route;  // FLN_ROUTE_*
-  int vec;    // elements per lane load (16 bytes on the vector path, 1 on the scalar path)
+  int vec;    // elements per lane load (16 bytes' worth; 1 on the scalar path)
   int cap, wide_cap;
   FwdGeometry g;
 };
@@ -1818,7 +1962,12 @@ FwdPlan plan_typed(int64_t rows, int64_t N, bool has_res, int gelu, bool vec_ok,
   constexpr int VV = 16 / sizeof(T);  // elements per 16-byte vector
   const Tuning& tun = tuning();
   FwdPlan pl{};
-  pl.vec = vec_ok ? VV : 1;
+  // Off the vector path's alignment, rows of more than kScalarCols columns are ragged: 16-byte
+  // vectors, unaligned.  Shorter ones would leave most lanes of a wave without a vector and take
+  // one element per lane (us, scalar / ragged: bf16 65536 x 65 14.8 / 18.9, x 100 14.8 / 18.5, x
+  // 333 27.5 / 23.2; fp32 65536 x 33 14.1 / 16.1).
+  const bool ragged = !vec_ok && N > kScalarCols;
+  pl.vec = vec_ok || ragged ? VV : 1;
   if (tun.force_loop || sizeof(T) == 8) {
     pl.route = FLN_ROUTE_LOOP;
     pl.g.loop = true;
@@ -1831,19 +1980,22 @@ FwdPlan plan_typed(int64_t rows, int64_t N, bool has_res, int gelu, bool vec_ok,
   // take up to 7 vectors (56 16-bit elements) per lane where they fill every lane.
   const int epl = tun.fwd_epl > 0 ? tun.fwd_epl : 32;
   int cap = (epl >= vec ? epl : vec) / vec;
-  const int max_cap = vec_ok ? max_vpl<VV>() : max_vpl<1>();
+  const int max_cap = vec == VV ? max_vpl<VV>() : max_vpl<1>();
   if (cap > max_cap) cap = max_cap;
-  // Rows of more than 4 waves: 16 elements per lane (8 on the scalar path) keep every flavour
-  // within the 128 VGPRs of a 1024-thread block.
-  int wide_cap = vec_ok ? 16 / VV : 8;
+  // Rows of more than 4 waves: 16 elements per lane keep every flavour within the 128 VGPRs of a
+  // 1024-thread block.
+  int wide_cap = vec == VV ? 16 / VV : max_cap;
   if (wide_cap > cap) wide_cap = cap;
   pl.cap = cap;
   pl.wide_cap = wide_cap;
   // The 32-element RAW tiles only for 16-bit types (fp32 ones would hold 64 VGPRs of gamma /
   // beta alone and spill); wider fp32 rows go to the LDS-staged kernel.
   const int raw_cap = (vec_ok && VV < 8) ? wide_cap : max_cap;
-  const int64_t nvec = N / vec;
-  FwdGeometry g = fwd_geometry(rows, nvec, cap, wide_cap, raw_cap, vec_ok, tun.fwd_wpr, cus);
+  const int64_t nvec = (N + vec - 1) / vec;
+  FwdGeometry g =
+      ragged ? ragged_geometry(rows, nvec, vec, gelu == FLN_GELU_ERF, tun.fwd_wpr, cus)
+             : fwd_geometry(rows, nvec, cap, wide_cap, raw_cap, vec_ok,
+                            vec == VV ? tun.fwd_wpr : 0, cus);
   // The fp8 row scale (no residual) and 16-bit LN + GELU take 4 waves per row with masked tail
   // lanes over an exact tiling of 5-7 waves when at most 1/8 of the 4-wave tile is masked (bf16,
   // 32768 x 7168 LN -> fp8: 7 waves 134.5 us at its best grid, 4 waves 129.9 us; 8192 x 7168
@@ -2086,13 +2238,16 @@ int dispatch_typed(FwdParams p, hipStream_t s) {
       if constexpr (FP8 == 0) return launch_lds_reg<T, VV>(p, s);
       return FLN_ERR_INVALID;  // not planned for fp8 outputs
     case FLN_ROUTE_WIDE:
-      return vec_ok ? launch_wide<T, FP8, VV>(p, s) : launch_wide<T, FP8, 1>(p, s);
+      return vec_ok ? launch_wide<T, FP8, VV, false>(p, s) : launch_wide<T, FP8, VV, true>(p, s);
     case FLN_ROUTE_LOOP: return launch_loop<T, float, FP8>(p, s);
     default: break;
   }
   p.wpr = pl.g.wpr;
-  if (vec_ok) return launch_reg_flavour<T, FP8, VV>(p, pl.g.vpl, pl.g.exact, pl.g.threads, s);
-  return launch_reg_flavour<T, FP8, 1>(p, pl.g.vpl, false, pl.g.threads, s);
+  if (pl.vec == VV) {
+    const int fit = !vec_ok ? kRaggedFit : pl.g.exact ? kExactFit : kMaskedFit;
+    return launch_reg_flavour<T, FP8, VV>(p, pl.g.vpl, fit, pl.g.threads, s);
+  }
+  return launch_reg_flavour<T, FP8, 1>(p, pl.g.vpl, kMaskedFit, pl.g.threads, s);
 }
 
 }  // namespace detail

@@ -1,0 +1,75 @@
+"""GPU parity of rows off the 16-byte grid: widths that are no whole number of 16-byte vectors and
+pointers off a 16-byte boundary, at the edges of their tiles, against the oracle's bars."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+import capi
+import test_gpu_capi as checks
+from gpu_calls import cuda, ln_forward, workspace
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float32, torch.bfloat16, torch.float16]
+KINDS = ["ln", "rms", "gelu_tanh", "gelu_none", "add_ln", "ln_fp8", "ln_dres", "add_rms",
+         "rms_fp8", "add_ln_fp8"]
+# One column past / short of a wave's, a tile's or a block's worth of vectors (16-bit and fp32),
+# with every remainder of a vector among them; 16383 the widest register rows.
+WIDTHS = [257, 263, 511, 513, 1030, 1281, 2049, 2561, 3071, 4097, 6145, 8191, 8193, 12292, 16383]
+ROWS = [1, 37, 600]
+
+
+@pytest.fixture(scope="module")
+def lib(gpu_available):
+    return capi.load()
+
+
+def _cases():
+    for i, cols in enumerate(WIDTHS):
+        for j, kind in enumerate(KINDS):
+            yield kind, DTYPES[(i + j) % 3], ROWS[(i + 2 * j) % 3], cols, (i + j) % 4 == 3
+    for i, cols in enumerate([288, 4096, 16384]):  # whole vectors and MX blocks, off alignment
+        for j, kind in enumerate(KINDS + ["ln_mx", "add_rms_mx"]):
+            yield kind, DTYPES[(i + j) % 3], ROWS[(i + j) % 3], cols, True
+
+
+@pytest.mark.parametrize("kind,dtype,rows,cols,shifted", list(_cases()),
+                         ids=lambda v: str(v)[6:] if isinstance(v, torch.dtype) else str(v))
+def test_ragged_rows(lib, kind, dtype, rows, cols, shifted):
+    """The forward (and backward, where the flavour has one) of ragged rows within the bars of
+    the random-shape test."""
+    checks.test_random_shapes_against_the_oracle(lib, kind, dtype, rows, cols, shifted)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("rows,cols", [(5, 1023), (300, 513), (2, 8193), (3, 20001)])
+def test_ragged_outputs_stay_inside(lib, dtype, rows, cols):
+    """y and dx inside larger buffers: not a byte before or after them changes."""
+    gen = torch.Generator().manual_seed(cols)
+    pad = 64
+    x, dy = (cuda(torch.randn(rows, cols, generator=gen).to(dtype)) for _ in range(2))
+    g = cuda(torch.randn(cols, generator=gen).to(dtype))
+    y0, mean, rstd = ln_forward(lib, x, g, None, 1e-5)
+    n = rows * cols
+    p = capi.ptr
+    code, st = capi.dtype_code(x), capi.stream()
+    ws, nb = workspace(lib, rows, cols, x)
+
+    def fwd(out):
+        return lib.fln_layernorm_forward(p(x), p(g), None, p(out), None, None, rows, cols, code,
+                                         1e-5, st)
+
+    def bwd(out):  # dx alone
+        return lib.fln_layernorm_backward(p(dy), p(x), p(mean), p(rstd), p(g), None, p(out), None,
+                                          None, rows, cols, code, capi.F32, p(ws), nb, st)
+
+    dx0 = torch.empty_like(x)
+    capi.check(bwd(dx0))
+    for lead in (1, pad):  # off and on a 16-byte boundary
+        for call, want in ((fwd, y0), (bwd, dx0)):
+            buf = torch.full((lead + n + pad,), 7.0, device="cuda", dtype=dtype)
+            out = buf[lead:lead + n]
+            capi.check(call(out))
+            assert (buf[:lead] == 7).all() and (buf[lead + n:] == 7).all()
+            assert torch.equal(out.view(rows, cols), want)
