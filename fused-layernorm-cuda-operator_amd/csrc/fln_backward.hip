@@ -120,6 +120,24 @@ __device__ __forceinline__ void reduce_quad_block(const ColReduceArgs& a, int64_
   __syncthreads();  // comb is reused by the caller's next quad block
 }
 
+// Column sums of a ragged row's vector, stored 16 bytes at a time at 4-byte alignment.  The columns
+// that a row's last vector shares with the one before it are written by both, with the same value
+// (the same rows summed in the same order).  Element by element behind a test of the shared ones,
+// each wave-wide store touched 32-byte strides: fp16 100 x 5001 backward 14.2 us against 10.7.
+template <int VEC> __device__ __forceinline__ void store_columns(float* out, const float* vals) {
+  struct __attribute__((packed, aligned(4))) Quad {
+    float v[4];
+  };
+  static_assert(VEC % 4 == 0, "whole quads");
+#pragma unroll
+  for (int k = 0; k < VEC / 4; ++k) {
+    Quad q;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q.v[e] = vals[4 * k + e];
+    *reinterpret_cast<Quad*>(out + 4 * k) = q;
+  }
+}
+
 // Rows in flight ahead of the current one.  Measured on MI355X over bf16 / fp16 / fp32 rows of
 // 768 to 16384 columns: 2 rows beat 1 and 3 when a lane holds one vector of a row; with two
 // vectors per lane (16-bit rows wider than 8192 columns, fp32 wider than 4096) a deeper ring no
@@ -141,7 +159,16 @@ __device__ __forceinline__ void reduce_quad_block(const ColReduceArgs& a, int64_
 // a = xhat gamma + beta is recomputed from the saved statistics, and dy is replaced by
 // dy GELU'(a) before the LayerNorm algebra (so dgamma / dbeta are sums of dy GELU'(a) xhat and
 // of dy GELU'(a)).
-template <class T, bool DRES, int GELU, int VEC, int VPL, int MAXT>
+// RAGGED: rows off the 16-byte grid (RaggedRow), up to 16384 columns of a 16-bit type and 8192 of
+// fp32, with unaligned 16-byte accesses, as in the forward.  Every 16 lanes' 256 bytes touch three
+// 128-byte lines instead of two, which bounds it (8192 x 4095 moves 4.8 TB/s, aligned 4096 columns
+// 5.05).  dx stores take the default policy: adjacent waves write parts of one line, which L2 then
+// merges (8192 x 4092 48.2 -> 45.7 us).  bf16 backward calls against the scalar path (one element
+// per lane and load), us: 8192 x 4095 52.1 -> 42.0, 4000 x 4097 39.6 -> 31.8, 16384 x 1023 31.6 ->
+// 25.4, 4000 x 9999 163.8 (two passes) -> 60.0; fp32 4000 x 5003 58.2 -> 48.1; erf GELU 14591 x 1146
+// 39.7 -> 30.2, 2000 x 13001 113.3 -> 57.1; residual gradient 4000 x 4097 46.3 -> 38.8.  The two
+// passes of wider rows: 2048 x 24001 191.3 -> 127.7, fp32 1000 x 20001 107.4 -> 87.6.
+template <class T, bool DRES, int GELU, int VEC, int VPL, int MAXT, bool RAGGED>
 __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
   constexpr int MAXW = MAXT / kWave;
   // RAW: 16-bit rows of 18433..24576 columns, 3 vectors per lane in a 1024-thread block.  The
@@ -154,6 +181,7 @@ __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
   // in flight while the next row loads).
   constexpr bool NOPF = RAW && VPL == 4;
   static_assert(!NOPF || (GELU == 0 && !DRES), "4-vector raw tiles: LayerNorm / RMSNorm only");
+  static_assert(!(RAGGED && RAW), "ragged rows: no raw tiles");
   constexpr int PD = NOPF ? 1 : FLN_BWD_PREFETCH(VPL);  // rows in flight ahead of the current one
 
   // [double buffer][sum g, sum g*xhat][wave], padded for combine_partials
@@ -171,6 +199,27 @@ __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
   const int64_t N = p.cols;
   const uint32_t row_bytes = static_cast<uint32_t>(N * sizeof(T));
   const float inv_n = 1.0f / static_cast<float>(N);
+  // Byte offset of this lane's vector slot i in a row.  A ragged row's last vector lies in a last
+  // slot (the dispatch picks the waves so).
+  const RaggedRow<T, VEC> rag(static_cast<uint32_t>(RAGGED ? N : VEC));
+  uint32_t rag_off[RAGGED ? VPL : 1];
+  uint32_t rag_own[RAGGED ? VEC : 1];  // all ones: element e of the last slot counts in row sums
+  if constexpr (RAGGED) {
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) rag_off[i] = rag.off(static_cast<uint32_t>(t + i * tpr));
+    const int lo = rag.lo(static_cast<uint32_t>(t + (VPL - 1) * tpr));
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      rag_own[e] = e >= lo ? 0xFFFFFFFFu : 0u;
+      asm volatile("" : "+v"(rag_own[e]));  // a VGPR each: as compares they spill SGPR pairs
+    }
+  }
+  auto off = [&](int i) -> uint32_t {
+    if constexpr (RAGGED)
+      return rag_off[i];
+    else
+      return static_cast<uint32_t>(t + i * tpr) * static_cast<uint32_t>(sizeof(P));
+  };
   // Rows are dealt out grid-stride: iteration `it` of block b handles row group
   // (it * gridDim.x + b), i.e. rows (it * gridDim.x + b) * rgs + rg.  At any moment all blocks
   // work on one window of adjacent rows, which keeps HBM page locality like a streaming copy;
@@ -203,7 +252,7 @@ __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
     const T one = from_f32<T>(1.0f);
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      P gv = buf_load<P>(gr, t + i * tpr);
+      P gv = buf_load_at<P>(gr, off(i));
 #pragma unroll
       for (int e = 0; e < VEC; ++e)
         if (!has_g) gv.v[e] = one;
@@ -217,9 +266,9 @@ __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
 #pragma unroll
       for (int i = 0; i < VPL; ++i) {
         if constexpr (PARAMS_IN_LDS)
-          bsh[i * MAXT + threadIdx.x] = buf_load<P>(br, t + i * tpr);
+          bsh[i * MAXT + threadIdx.x] = buf_load_at<P>(br, off(i));
         else
-          btr[i] = buf_load<P>(br, t + i * tpr);
+          btr[i] = buf_load_at<P>(br, off(i));
       }
     }
   }
@@ -259,13 +308,13 @@ __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
     const rsrc_t dr = make_rsrc(DY + row * N, nb);
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      xn[slot][i] = buf_load<P, FLN_BWD_LOAD_POL>(xr, t + i * tpr);
-      dn[slot][i] = buf_load<P, FLN_BWD_LOAD_POL>(dr, t + i * tpr);
+      xn[slot][i] = buf_load_at<P, FLN_BWD_LOAD_POL>(xr, off(i));
+      dn[slot][i] = buf_load_at<P, FLN_BWD_LOAD_POL>(dr, off(i));
     }
     if constexpr (DRES) {
       const rsrc_t rr = make_rsrc(DR + row * N, nb);
 #pragma unroll
-      for (int i = 0; i < VPL; ++i) rn[slot][i] = buf_load<P, FLN_BWD_LOAD_POL>(rr, t + i * tpr);
+      for (int i = 0; i < VPL; ++i) rn[slot][i] = buf_load_at<P, FLN_BWD_LOAD_POL>(rr, off(i));
     }
     const uint32_t sb = nb ? 4u : 0u;
     mun[slot] = __builtin_bit_cast(
@@ -395,8 +444,13 @@ __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         gd[i][e] = DD(i, e) * gam(i, e);
-        s1 += gd[i][e];
-        s2 = fmaf(gd[i][e], XH(i, e), s2);
+        float g = gd[i][e];
+        if constexpr (RAGGED) {  // the last vector counts only its own elements
+          if (i == VPL - 1)
+            g = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, g) & rag_own[e]);
+        }
+        s1 += g;
+        s2 = fmaf(g, XH(i, e), s2);
       }
     // RAW: the packs become opaque here, so that dx widens them again rather than the compiler
     // keeping the fp32 values of the row sums alive across the reduction.
@@ -438,7 +492,7 @@ __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
       }
     const rsrc_t xo = make_rsrc(DX ? DX + row * N : nullptr, nb);
 #pragma unroll
-    for (int i = 0; i < VPL; ++i) buf_store<P, FLN_BWD_STORE_POL>(o[i], xo, t + i * tpr);
+    for (int i = 0; i < VPL; ++i) buf_store_at<P, RAGGED ? kDefault : FLN_BWD_STORE_POL>(o[i], xo, off(i));
     // The next step's (cheap) widening must not be hoisted above this step's loads and stores.
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -446,7 +500,7 @@ __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
 
   // Stage-1 output: one fp32 partial row per block (row stride ld, a multiple of 4).
   const int64_t ld = (N + 3) & ~int64_t(3);
-  const int nvec = static_cast<int>(N / VEC);
+  const int nvec = RAGGED ? static_cast<int>(rag.nvec) : static_cast<int>(N / VEC);
   float* outs[2] = {p.part_g, p.part_b};
 #pragma unroll
   for (int a = 0; a < 2; ++a) {
@@ -471,8 +525,12 @@ __global__ __launch_bounds__(MAXT) void bwd_reg_kernel(const BwdParams p) {
         }
       }
       if (rg == 0 && v < nvec) {
+        if constexpr (RAGGED) {
+          store_columns<VEC>(out + off(i) / static_cast<uint32_t>(sizeof(T)), vals);
+        } else {
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) out[static_cast<int64_t>(v) * VEC + e] = vals[e];
+          for (int e = 0; e < VEC; ++e) out[static_cast<int64_t>(v) * VEC + e] = vals[e];
+        }
       }
     }
   }
@@ -667,7 +725,7 @@ __global__ __launch_bounds__(NT) void bwd_lds_kernel(const BwdParams p) {
 
 // Rows past the register and LDS tiles (16-bit rows of more than 18432 columns, save the rows
 // of up to 24576 without a residual gradient (raw tiles); fp32 rows of more than 16384; long
-// rows on the scalar path), any width, in two streaming passes:
+// ragged rows), any width, in two streaming passes:
 //   bwd_rowstat_kernel: per row and column split, sum(g) and sum(g xhat) (g = dy' gamma,
 //     dy' = dy or dy GELU'(xhat gamma + beta)) into stats[row, split]; one 256-thread block per
 //     (row, split) at a time, grid-stride, eight vectors per thread in flight per array.  Few
@@ -698,7 +756,7 @@ constexpr int kMaxStatSplits = 16;
 #define FLN_COLPASS_BLOCKS_PER_CU 2
 #endif
 
-template <class T, int GELU, int VEC>
+template <class T, int GELU, int VEC, bool RAGGED>
 __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdParams p,
                                                                    float2* stats) {
   using P = Pack<T, VEC>;
@@ -708,7 +766,8 @@ __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdPara
   const int lane = t & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int64_t N = p.cols;
-  const int nvec = static_cast<int>(N / VEC);
+  const RaggedRow<T, VEC> rag(static_cast<uint32_t>(RAGGED ? N : VEC));
+  const int nvec = RAGGED ? static_cast<int>(rag.nvec) : static_cast<int>(N / VEC);
   const uint32_t row_bytes = static_cast<uint32_t>(N * sizeof(T));
   const T* X = static_cast<const T*>(p.x);
   const T* DY = static_cast<const T*>(p.dy);
@@ -723,7 +782,8 @@ __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdPara
     const int64_t v_lo = (item - row * S) * p.stat_chunk;
     const int64_t v_hi = v_lo + p.stat_chunk < nvec ? v_lo + p.stat_chunk : nvec;
     // x and dy read as zeros past the split (g = 0 there), gamma / beta over the whole row.
-    const uint32_t split_bytes = static_cast<uint32_t>(v_hi * VEC * sizeof(T));
+    const uint32_t split_bytes =
+        RAGGED ? row_bytes : static_cast<uint32_t>(v_hi * VEC * sizeof(T));
     const rsrc_t xr = make_rsrc(X + row * N, split_bytes);
     const rsrc_t dr = make_rsrc(DY + row * N, split_bytes);
     const float mu = p.rms ? 0.0f : p.mean[row];
@@ -734,13 +794,22 @@ __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdPara
 #pragma unroll
       for (int u = 0; u < kWideUnroll; ++u) {  // vectors past the row read as zeros
         const int v = v0 + u * kWideThreads;
-        xv[u] = buf_load<P, kStream>(xr, v);
-        dv[u] = buf_load<P, kStream>(dr, v);
-        gv[u] = buf_load<P>(gr, v);
-        if constexpr (GELU != 0) bv[u] = buf_load<P>(br, v);
+        const uint32_t o = !RAGGED   ? static_cast<uint32_t>(v) * static_cast<uint32_t>(sizeof(P))
+                           : v < v_hi ? rag.off(static_cast<uint32_t>(v))
+                                      : kOutOfRange;
+        xv[u] = buf_load_at<P, kStream>(xr, o);
+        dv[u] = buf_load_at<P, kStream>(dr, o);
+        gv[u] = buf_load_at<P>(gr, o);
+        if constexpr (GELU != 0) bv[u] = buf_load_at<P>(br, o);
       }
 #pragma unroll
-      for (int u = 0; u < kWideUnroll; ++u)
+      for (int u = 0; u < kWideUnroll; ++u) {
+        // A ragged row's last vector counts only its own elements.
+        if (RAGGED && v0 + u * kWideThreads == nvec - 1) {
+#pragma unroll
+          for (int e = 0; e < VEC; ++e)
+            if (e < static_cast<int>(rag.dup)) dv[u].v[e] = from_f32<T>(0.0f);
+        }
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           const float xh = (to_f32(xv[u].v[e]) - mu) * rs;
@@ -752,6 +821,7 @@ __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdPara
           s1 += g;
           s2 = fmaf(g, xh, s2);
         }
+      }
     }
     s1 = wave_allreduce<SumOp>(s1);
     s2 = wave_allreduce<SumOp>(s2);
@@ -767,13 +837,16 @@ __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdPara
   }
 }
 
-template <class T, bool DRES, int GELU, int VEC>
+template <class T, bool DRES, int GELU, int VEC, bool RAGGED>
 __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdParams p,
                                                                    const float2* stats) {
   using P = Pack<T, VEC>;
   const int v = blockIdx.x * kWideThreads + threadIdx.x;  // this thread's vector column
   const int64_t N = p.cols;
-  const int nvec = static_cast<int>(N / VEC);
+  const RaggedRow<T, VEC> rag(static_cast<uint32_t>(RAGGED ? N : VEC));
+  const int nvec = RAGGED ? static_cast<int>(rag.nvec) : static_cast<int>(N / VEC);
+  const uint32_t off = RAGGED ? rag.off(static_cast<uint32_t>(v))
+                              : static_cast<uint32_t>(v) * static_cast<uint32_t>(sizeof(P));
   const uint32_t row_bytes = static_cast<uint32_t>(N * sizeof(T));
   const float inv_n = 1.0f / static_cast<float>(N);
   // Block y takes rows y, y + G, y + 2G, ... (G = gridDim.y): all blocks stream through one
@@ -784,12 +857,12 @@ __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdPara
   const T* DY = static_cast<const T*>(p.dy);
   const T* DR = static_cast<const T*>(p.dres);
   T* DX = static_cast<T*>(p.dx);
-  P gv = buf_load<P>(make_rsrc(p.gamma, row_bytes), v);
+  P gv = buf_load_at<P>(make_rsrc(p.gamma, row_bytes), off);
   if (p.gamma == nullptr)
 #pragma unroll
     for (int e = 0; e < VEC; ++e) gv.v[e] = from_f32<T>(1.0f);
   P bv{};
-  if constexpr (GELU != 0) bv = buf_load<P>(make_rsrc(p.beta, row_bytes), v);
+  if constexpr (GELU != 0) bv = buf_load_at<P>(make_rsrc(p.beta, row_bytes), off);
   float acc_g[VEC], acc_b[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) acc_g[e] = acc_b[e] = 0.0f;
@@ -803,9 +876,9 @@ __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdPara
       const bool in = row + u * G < p.rows;  // uniform
       const int64_t r = in ? row + u * G : row;
       const uint32_t nb = in ? row_bytes : 0u;
-      xv[u] = buf_load<P, kStream>(make_rsrc(X + r * N, nb), v);
-      dv[u] = buf_load<P, kStream>(make_rsrc(DY + r * N, nb), v);
-      if constexpr (DRES) rv[u] = buf_load<P, kStream>(make_rsrc(DR + r * N, nb), v);
+      xv[u] = buf_load_at<P, kStream>(make_rsrc(X + r * N, nb), off);
+      dv[u] = buf_load_at<P, kStream>(make_rsrc(DY + r * N, nb), off);
+      if constexpr (DRES) rv[u] = buf_load_at<P, kStream>(make_rsrc(DR + r * N, nb), off);
       mu[u] = p.rms ? 0.0f : p.mean[r];
       rs[u] = p.rstd[r];
       // The row's splits: lane k of each 16-lane row loads split k.
@@ -837,21 +910,30 @@ __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdPara
           acc_b[e] += d;
         }
       }
-      buf_store<P, kStream>(o, make_rsrc(DX ? DX + r * N : nullptr, in ? row_bytes : 0u), v);
+      buf_store_at<P, kStream>(o, make_rsrc(DX ? DX + r * N : nullptr, in ? row_bytes : 0u), off);
     }
   }
   if (v >= nvec) return;
+  // (A ragged row's last vector writes the columns it shares with the vector before it as well:
+  // the same sums.)
+  const int64_t col = RAGGED ? static_cast<int64_t>(off / static_cast<uint32_t>(sizeof(T)))
+                             : static_cast<int64_t>(v) * VEC;
   if (p.out_g != nullptr || p.out_b != nullptr) {  // one block row: these sums are final
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      const int64_t j = static_cast<int64_t>(v) * VEC + e;
+      const int64_t j = col + e;
       if (p.out_g) store_param(p.out_g, p.out_dtype, j, acc_g[e]);
       if (p.out_b) store_param(p.out_b, p.out_dtype, j, acc_b[e]);
     }
     return;
   }
   const int64_t ld = (N + 3) & ~int64_t(3);
-  const int64_t c = static_cast<int64_t>(blockIdx.y) * ld + static_cast<int64_t>(v) * VEC;
+  const int64_t c = static_cast<int64_t>(blockIdx.y) * ld + col;
+  if constexpr (RAGGED) {
+    if (p.part_g) store_columns<VEC>(p.part_g + c, acc_g);
+    if (p.part_b) store_columns<VEC>(p.part_b + c, acc_b);
+    return;
+  }
 #pragma unroll
   for (int e = 0; e < VEC; ++e) {
     if (p.part_g) p.part_g[c + e] = acc_g[e];
@@ -977,8 +1059,11 @@ __global__ __launch_bounds__(kCrFlatThreads) void col_reduce_flat_kernel(const C
 namespace {
 
 // Largest vectors per lane instantiated for the backward register path: 2 vectors (16
-// elements of a 16-bit type, 8 of fp32) on the vector path, 8 on the scalar path.
-constexpr int bwd_max_vpl(int vec, int es) { return vec == 1 ? 8 : 2; }
+// elements of a 16-bit type, 8 of fp32) on the vector path, 4 on the scalar path.
+constexpr int bwd_max_vpl(int vec, int es) { return vec == 1 ? 4 : 2; }
+// Rows off the vector path's alignment: up to this many columns they take the scalar path, more
+// are ragged (unaligned 16-byte vectors), as in the forward.
+constexpr int64_t kScalarCols = 256;
 // 16-bit rows of 16385..18432 columns: one row per 768-thread block, 3 vectors per lane.
 constexpr int kReg3Threads = 768;
 
@@ -990,10 +1075,10 @@ int next_pow2(int v) {
 
 // Stage-1 launch (resident == nullptr) or, with `resident`, the number of blocks of that
 // instantiation that fit on the device at once (occupancy x CUs, cached per device).
-template <class T, bool DRES, int GELU, int VEC, int VPL, int MAXT>
+template <class T, bool DRES, int GELU, int VEC, int VPL, int MAXT, bool RAGGED = false>
 int launch_stage1_k(const BwdParams& p, int64_t blocks, int threads, hipStream_t s,
                     int64_t* resident) {
-  auto kernel = bwd_reg_kernel<T, DRES, GELU, VEC, VPL, MAXT>;
+  auto kernel = bwd_reg_kernel<T, DRES, GELU, VEC, VPL, MAXT, RAGGED>;
   // The GELU kernels fill their LDS table with one entry per thread.
   if (GELU != 0 && threads < kGeluTabN) return FLN_ERR_INVALID;
   if (resident) {
@@ -1013,6 +1098,25 @@ int launch_stage1_k(const BwdParams& p, int64_t blocks, int threads, hipStream_t
   }
   static std::atomic<void*> fn_cache[64];
   return launch_cached(kernel, fn_cache, dim3(blocks), dim3(threads), s, p);
+}
+
+// Ragged rows: 1 or 2 vectors per lane of 1024-thread blocks.
+template <class T, int VEC>
+int launch_stage1_ragged(const BwdParams& p, int vpl, int64_t blocks, int threads, hipStream_t s,
+                         int64_t* resident) {
+  auto run = [&](auto n) {
+    constexpr int VPL = decltype(n)::value;
+    if (p.gelu == 1)
+      return launch_stage1_k<T, false, 1, VEC, VPL, 1024, true>(p, blocks, threads, s, resident);
+    if (p.gelu == 2)
+      return launch_stage1_k<T, false, 2, VEC, VPL, 1024, true>(p, blocks, threads, s, resident);
+    if (p.dres)
+      return launch_stage1_k<T, true, 0, VEC, VPL, 1024, true>(p, blocks, threads, s, resident);
+    return launch_stage1_k<T, false, 0, VEC, VPL, 1024, true>(p, blocks, threads, s, resident);
+  };
+  if (vpl == 1) return run(std::integral_constant<int, 1>{});
+  if (vpl == 2) return run(std::integral_constant<int, 2>{});
+  return FLN_ERR_INVALID;
 }
 
 template <class T, int VEC, int VPL>
@@ -1081,34 +1185,31 @@ int launch_stage1_vpl(const BwdParams& p, int vpl, int64_t blocks, int threads, 
       if constexpr (CAP >= 4 || VEC * sizeof(T) == 16)
         return launch_stage1<T, VEC, 4>(p, blocks, threads, s, resident);
       return FLN_ERR_INVALID;
-    case 8:
-      if constexpr (CAP >= 8) return launch_stage1<T, VEC, 8>(p, blocks, threads, s, resident);
-      return FLN_ERR_INVALID;
     default: return FLN_ERR_INVALID;
   }
 }
 
-template <class T, int VEC>
+template <class T, int VEC, bool RAGGED>
 int launch_two_pass(const BwdParams& p, const BwdGeometry& geo, hipStream_t s) {
   float2* stats = reinterpret_cast<float2*>(p.rowstat);
   const int64_t cap = kRowstatBlocksPerCu * static_cast<int64_t>(device_cu_count());
   const int64_t items = p.rows * p.stat_splits;
   const dim3 g1(static_cast<unsigned>(items < cap ? items : cap)), blk(kWideThreads);
-  const int64_t nvec = p.cols / VEC;
+  const int64_t nvec = (p.cols + VEC - 1) / VEC;
   const dim3 g2(static_cast<unsigned>((nvec + kWideThreads - 1) / kWideThreads),
                 static_cast<unsigned>(geo.blocks));
   if (p.gelu == 1) {
-    hipLaunchKernelGGL((bwd_rowstat_kernel<T, 1, VEC>), g1, blk, 0, s, p, stats);
-    hipLaunchKernelGGL((bwd_colpass_kernel<T, false, 1, VEC>), g2, blk, 0, s, p, stats);
+    hipLaunchKernelGGL((bwd_rowstat_kernel<T, 1, VEC, RAGGED>), g1, blk, 0, s, p, stats);
+    hipLaunchKernelGGL((bwd_colpass_kernel<T, false, 1, VEC, RAGGED>), g2, blk, 0, s, p, stats);
   } else if (p.gelu == 2) {
-    hipLaunchKernelGGL((bwd_rowstat_kernel<T, 2, VEC>), g1, blk, 0, s, p, stats);
-    hipLaunchKernelGGL((bwd_colpass_kernel<T, false, 2, VEC>), g2, blk, 0, s, p, stats);
+    hipLaunchKernelGGL((bwd_rowstat_kernel<T, 2, VEC, RAGGED>), g1, blk, 0, s, p, stats);
+    hipLaunchKernelGGL((bwd_colpass_kernel<T, false, 2, VEC, RAGGED>), g2, blk, 0, s, p, stats);
   } else {
-    hipLaunchKernelGGL((bwd_rowstat_kernel<T, 0, VEC>), g1, blk, 0, s, p, stats);
+    hipLaunchKernelGGL((bwd_rowstat_kernel<T, 0, VEC, RAGGED>), g1, blk, 0, s, p, stats);
     if (p.dres)
-      hipLaunchKernelGGL((bwd_colpass_kernel<T, true, 0, VEC>), g2, blk, 0, s, p, stats);
+      hipLaunchKernelGGL((bwd_colpass_kernel<T, true, 0, VEC, RAGGED>), g2, blk, 0, s, p, stats);
     else
-      hipLaunchKernelGGL((bwd_colpass_kernel<T, false, 0, VEC>), g2, blk, 0, s, p, stats);
+      hipLaunchKernelGGL((bwd_colpass_kernel<T, false, 0, VEC, RAGGED>), g2, blk, 0, s, p, stats);
   }
   return static_cast<int>(hipGetLastError());
 }
@@ -1166,8 +1267,9 @@ int dispatch_backward(BwdParams p, const BwdGeometry& geo, hipStream_t s,
       *resident = geo.blocks;  // partial rows = row chunks of the column pass
       return 0;
     }
-    if (geo.vec == VV) return launch_two_pass<T, VV>(p, geo, s);
-    return launch_two_pass<T, 1>(p, geo, s);
+    if (geo.vec != VV) return FLN_ERR_INVALID;  // scalar rows fit the register path
+    if (geo.ragged) return launch_two_pass<T, VV, true>(p, geo, s);
+    return launch_two_pass<T, VV, false>(p, geo, s);
   }
   if (!geo.reg_path) {
     if (resident) {
@@ -1177,6 +1279,8 @@ int dispatch_backward(BwdParams p, const BwdGeometry& geo, hipStream_t s,
     hipLaunchKernelGGL((bwd_loop_kernel<T>), dim3(geo.blocks), dim3(1024), 0, s, p);
     return static_cast<int>(hipGetLastError());
   }
+  if (geo.ragged)
+    return launch_stage1_ragged<T, VV>(p, geo.vpl, geo.blocks, geo.threads, s, resident);
   if (geo.vec == VV)
     return launch_stage1_vpl<T, VV>(p, geo.vpl, geo.blocks, geo.threads, s, resident);
   return launch_stage1_vpl<T, 1>(p, geo.vpl, geo.blocks, geo.threads, s, resident);
@@ -1194,8 +1298,10 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   BwdGeometry g{};
   const int es = element_size(dtype);
   const int vv = es > 0 ? 16 / es : 1;
-  g.vec = (vec_ok && cols % vv == 0) ? vv : 1;
-  const int64_t nvec = cols / g.vec;
+  const bool aligned = vec_ok && cols % vv == 0;
+  g.ragged = !aligned && cols > kScalarCols;
+  g.vec = aligned || g.ragged ? vv : 1;
+  const int64_t nvec = (cols + g.vec - 1) / g.vec;
   auto per_lane = [&](int w) { return (nvec + kWave * w - 1) / (kWave * w); };
   // Elements per lane: 8 by default (x-hat, dy, g, gamma, both column accumulators and the
   // prefetched raw rows of a lane's columns stay in registers: 84-98 VGPRs for fp32 rows at 2
@@ -1213,15 +1319,35 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   while (per_lane(wpr) > cap && wpr < 16) wpr *= 2;
   if (per_lane(wpr) > cap) cap = bwd_max_vpl(g.vec, es);
   const int forced = tun.bwd_wpr;
-  if (forced >= 1 && forced <= 16 && (forced & (forced - 1)) == 0 && per_lane(forced) <= cap)
+  if (g.ragged) {
+    // Ragged rows: 1 or 2 vectors per lane over as many waves as that takes (at most 16), so that
+    // the row's last vector lies in a lane's last slot.  Two in 16-bit rows of more than 384 vectors
+    // where that masks at most 1/8 more slots (bf16 backward calls, us, waves x vectors: 4000 x
+    // 4097 5 x 2 34.5, 9 x 1 37.9; 6000 x 6001 6 x 2 55.3, 12 x 1 62.1; 4096 x 4095 4 x 2 30.1,
+    // 8 x 1 30.7; with a residual gradient 4000 x 4097 41.6 / 44.3; kept: 9000 x 2050 5 x 1 35.2, 3
+    // x 2 37.6; 16384 x 1023 2 x 1 24.4, 1 x 2 26.3; 14591 x 1146 GELU 3 x 1 29.7, 2 x 2 42.2),
+    // and in fp32 rows unless they are few (even: 3000 x 3003 25.5 for any tile).
+    const int64_t w1 = per_lane(1), w2 = (w1 + 1) / 2;
+    bool two = w1 > 16;
+    if (es == 2)
+      two = two || (!gelu && w2 >= 4 && w2 * 16 <= w1 * 9);
+    else
+      two = two || rows >= 4 * static_cast<int64_t>(device_cu_count());
+    cap = bwd_max_vpl(g.vec, es);
+    wpr = static_cast<int>(two ? w2 : w1);
+    if (forced >= 1 && forced <= 16 && per_lane(forced) <= cap) wpr = forced;
+    if (wpr > 16) wpr = 16;  // too wide: per_lane > cap, no register path
+  } else if (forced >= 1 && forced <= 16 && (forced & (forced - 1)) == 0 &&
+             per_lane(forced) <= cap) {
     wpr = forced;
+  }
   // 16-bit rows of 9-12 whole waves of vectors (4608-6144 columns) take a row group of exactly
   // that many waves instead of 16 with 4-7 of them idle.  bf16 backward calls, us, 8192 rows:
   // 4608 49.4 -> 44.8, 5120 50.6 -> 49.0, 5632 56.7 -> 53.4, 6144 59.6 -> 57.1 (16384 rows:
   // 5120 87.9 / 88.1, 6144 105.8 -> 104.1).  Fewer waves than 9 in a power-of-two group lost
   // (16384 x 2560, 5 of 8 waves: 47.8 -> 48.8; 32768 x 1536, 3 of 4: 55.3 -> 55.9), 14 of 16
   // tied (8192 x 7168 66.5 / 66.6).
-  if (es == 2 && g.vec == 8 && wpr == 16 && cap == 1 && nvec % kWave == 0 &&
+  if (es == 2 && g.vec == 8 && !g.ragged && wpr == 16 && cap == 1 && nvec % kWave == 0 &&
       nvec / kWave >= 9 && nvec / kWave <= 12 && forced <= 0)
     wpr = static_cast<int>(nvec / kWave);
   // 16-bit LayerNorm / RMSNorm rows whose one-vector tile leaves lanes masked (768, 1280, 1536,
@@ -1234,7 +1360,7 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   // 16384 x 2048 38.44 / 38.65, 8192 x 4096 39.84 / 40.50), and so do the GELU flavours, whose
   // 2-vector tiles keep gamma / beta in LDS (16384 x 768 tanh 22.4 -> 25.1, 16384 x 3072 erf
   // 63.4 -> 68.8).
-  if (es == 2 && g.vec == 8 && cap == 1 && forced <= 0 && tun.bwd_epl <= 0 && !gelu && !dres &&
+  if (es == 2 && g.vec == 8 && !g.ragged && cap == 1 && forced <= 0 && tun.bwd_epl <= 0 && !gelu && !dres &&
       nvec % (static_cast<int64_t>(kWave) * wpr) != 0 && rows >= 16 * device_cu_count()) {
     cap = 2;
     wpr = 1;
@@ -1256,6 +1382,8 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   if (tun.bwd_threads <= 0 && g.reg_path) {
     for (int t = 256; t < 1024; t *= 2) {
       if (t < kWave * g.wpr) continue;
+      // The GELU kernels fill their LDS table with one entry per thread.
+      if (gelu && t / (kWave * g.wpr) * (kWave * g.wpr) < kGeluTabN) continue;
       const int per_block = t / (kWave * g.wpr);
       if ((rows + per_block - 1) / per_block <= device_cu_count()) {
         threads = t;
@@ -1273,7 +1401,9 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
       const int64_t moved = cols * es * (dres ? 4 : 3);
       const int64_t target = gelu ? (48 << 10) : (24 << 10);
       threads = 1024;
-      if (512 >= kWave * g.wpr && (512 / (kWave * g.wpr)) * moved >= target) threads = 512;
+      // (Ragged rows: at least two row groups, 4000 x 4097 in 5 waves 35.7 -> 34.5.)
+      const int groups = 512 / (kWave * g.wpr);
+      if (groups >= (g.ragged ? 2 : 1) && groups * moved >= target) threads = 512;
     }
   }
   if (!g.reg_path) threads = 1024;
@@ -1299,7 +1429,7 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   // 115.0, GELU erf 145.8 -> 99.3, tanh 147.9 -> 99.2; 300 x 18432 LN 42.6 -> 26.6.  fp16 with a
   // residual gradient spills there (52 B per lane) and keeps the LDS-staged kernel (130.2
   // against 129.3 us).
-  if (!g.reg_path && es == 2 && g.vec == 8 && nvec > 2 * 1024 && nvec <= 3 * kReg3Threads &&
+  if (!g.reg_path && es == 2 && g.vec == 8 && !g.ragged && nvec > 2 * 1024 && nvec <= 3 * kReg3Threads &&
       !(dres && dtype == FLN_F16) && tun.bwd_no_lds == 0) {
     g.reg_path = true;
     g.vpl = 3;
@@ -1316,7 +1446,7 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   // 161.4 -> 117.5), 2048 x 19000 93.0 -> 63.2, 300 x 24576 56.1 -> 32.5; the GELU flavours
   // against the two passes (68 B of spill left): 4096 x 20480 erf 220.8 -> 184.3, tanh 201.1
   // -> 184.0, 4096 x 24576 erf 243.8 -> 197.3.
-  if (!g.reg_path && es == 2 && g.vec == 8 && nvec > 3 * kReg3Threads && nvec <= 3 * 1024 &&
+  if (!g.reg_path && es == 2 && g.vec == 8 && !g.ragged && nvec > 3 * kReg3Threads && nvec <= 3 * 1024 &&
       !dres && tun.bwd_no_lds == 0) {
     g.reg_path = true;
     g.vpl = 3;
@@ -1332,7 +1462,7 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   // 12288 LN 113.5 -> 108.6, RMSNorm 108.5 -> 105.4, GELU erf 121.4 -> 118.0, + residual 149.4
   // -> 144.3, 2048 x 12288 tanh 71.2 -> 68.2, 300 x 12288 28.9 -> 24.6; 4096 x 16384 LN 153.9
   // -> 147.0, RMSNorm 147.1 -> 142.2, 300 x 16384 33.9 -> 31.2.
-  if (!g.reg_path && es == 4 && g.vec == 4 && nvec > 2 * 1024 &&
+  if (!g.reg_path && es == 4 && g.vec == 4 && !g.ragged && nvec > 2 * 1024 &&
       (nvec <= 3 * 1024 || (nvec <= 4 * 1024 && !dres && !gelu)) && tun.bwd_no_lds == 0) {
     g.reg_path = true;
     g.vpl = nvec <= 3 * 1024 ? 3 : 4;
@@ -1349,7 +1479,7 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   // 99.9 -> 91.8, RMSNorm 2048 x 28672 121.2 -> 92.2, fp16 2048 x 32768 124.5 -> 105.9; with
   // fewer rows the two passes win (1024 x 32768 71.6 against 74.0, 300 x 32768 37.2 against
   // 49.0).
-  if (!g.reg_path && es == 2 && g.vec == 8 && nvec > 3 * 1024 && nvec <= 4 * 1024 && !dres &&
+  if (!g.reg_path && es == 2 && g.vec == 8 && !g.ragged && nvec > 3 * 1024 && nvec <= 4 * 1024 && !dres &&
       !gelu && rows >= 6 * int64_t(device_cu_count()) && tun.bwd_no_lds == 0) {
     g.reg_path = true;
     g.vpl = 4;
@@ -1370,7 +1500,7 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   const int64_t cpt16 = (nvec + kLds16Threads - 1) / kLds16Threads;
   const bool wide_f32 = !g.reg_path && es == 4 && cpt >= 3 && cpt <= 4;
   const bool wide16 = !g.reg_path && es == 2 && !gelu && cpt16 == 3 && dres && dtype == FLN_F16;
-  if (g.vec > 1 && (wide_f32 || wide16) && tun.bwd_no_lds == 0) {
+  if (g.vec > 1 && !g.ragged && (wide_f32 || wide16) && tun.bwd_no_lds == 0) {
     g.reg_path = false;
     g.lds_cpt = wide16 ? static_cast<int>(cpt16) : static_cast<int>(cpt);
     g.threads = wide16 ? kLds16Threads : kLdsThreads;
@@ -1442,7 +1572,7 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
   // with it the summation order never depend on the caller's workspace) leaves after the
   // partials.
   int64_t splits = 1;
-  const int64_t nvec = p.cols / geo.vec;
+  const int64_t nvec = (p.cols + geo.vec - 1) / geo.vec;
   p.stat_chunk = nvec;
   if (geo.two_pass) {
     constexpr int64_t step = int64_t(kWideUnroll) * kWideThreads;
