@@ -9,11 +9,14 @@
 #include <torch/extension.h>
 #include <torch/library.h>
 
+#include <ATen/core/dispatch/Dispatcher.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <array>
 #include <mutex>
@@ -675,6 +678,251 @@ Tensor rms_norm_autograd(const Tensor& input, int64_t normalized, const OptT& we
   return y;
 }
 
+// ------------------------------------------------------------------------------------------
+// The eager path of the other differentiable calls: LayerNorm and RMSNorm over several trailing
+// dimensions, LayerNorm + GELU, residual add + LayerNorm / RMSNorm.  Through the operators, each
+// costs a Python autograd Function in both directions, views of every argument, and zero-filled
+// gradients for the statistics outputs (a training step of 8 x 768 rows, host-bound, us:
+// layer_norm_gelu 155, add_rms_norm 148, FusedLayerNorm over [64, 32, 32] 143; nn.LayerNorm 73).
+// Here one node holds what the operators' formulas save (the normalized rows, weight, bias, mean,
+// rstd) and its backward calls the same functions, so outputs and gradients are the same bits.
+// ------------------------------------------------------------------------------------------
+enum NormKind { kLayerNorm = 0, kRmsNorm = 1, kLayerNormGelu = 2, kAddLayerNorm = 3, kAddRmsNorm = 4 };
+
+// Whether a call on these tensors may pass the dispatcher by: ordinary GPU tensors, nothing that
+// watches or rewrites operator calls (dispatch modes, tracing, functorch transforms, subclasses),
+// no forward-mode tangents.
+bool plain_call(std::initializer_list<const Tensor*> tensors) {
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing() ||
+      c10::impl::tls_local_dispatch_key_set().included_.has(
+          c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+    return false;
+  constexpr c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::Functionalize,
+                                         c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::FuncTorchBatched,
+                                         c10::DispatchKey::Batched, c10::DispatchKey::Conjugate,
+                                         c10::DispatchKey::Negative});
+  for (const Tensor* t : tensors) {
+    if (t == nullptr || !t->defined()) continue;
+    if (!t->is_cuda() || t->layout() != at::kStrided || t->key_set().has_any(special) ||
+        t->_fw_grad(0).defined())
+      return false;
+  }
+  return true;
+}
+
+// The [rows, n] form of a contiguous tensor, and a 1-D form of a parameter.
+Tensor as_rows(const Tensor& t, int64_t n) {
+  return t.dim() == 2 && t.size(1) == n ? t : t.view({t.numel() / n, n});
+}
+OptT as_param(const OptT& p) {
+  return has(p) && p->dim() != 1 ? OptT(p->reshape({-1})) : p;
+}
+
+struct FusedNormBackward : public torch::autograd::Node {
+  torch::autograd::SavedVariable rows_, w_, b_, mean_, rstd_;  // rows_: the input, or h
+  NormKind kind = kLayerNorm;
+  int64_t n = 0;
+  std::string approximate;
+  bool has_w = false, has_b = false;
+
+  // A registered backward operator by name, or the function itself where nothing watches.
+  template <class Fn, class... Args>
+  static auto call(bool direct, const char* op, Fn* fn, Args&&... args) {
+    if (direct) return fn(std::forward<Args>(args)...);
+    return c10::Dispatcher::singleton()
+        .findSchemaOrThrow(op, "")
+        .template typed<Fn>()
+        .call(std::forward<Args>(args)...);
+  }
+
+  torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    const bool add = kind == kAddLayerNorm || kind == kAddRmsNorm;
+    const bool rms = kind == kRmsNorm || kind == kAddRmsNorm;
+    torch::autograd::variable_list out(4);
+    Tensor gy = grads[0], gh = add ? grads[1] : Tensor();
+    const bool need_x = task_should_compute_output(0) || (add && task_should_compute_output(1));
+    const bool need_w = has_w && task_should_compute_output(2);
+    const bool need_b = has_b && task_should_compute_output(3);
+    if ((!gy.defined() && !gh.defined()) || !(need_x || need_w || need_b)) return out;
+    const Tensor rows = add ? rows_.unpack(shared_from_this()) : rows_.unpack();
+    const Tensor rstd = rstd_.unpack(), mean = rms ? Tensor() : mean_.unpack();
+    const OptT w = has_w ? OptT(w_.unpack()) : std::nullopt;
+    const OptT b = has_b ? OptT(b_.unpack()) : std::nullopt;
+    // Differentiating this backward, or a mode or subclass that looks on: the operators.
+    const bool direct =
+        !c10::GradMode::is_enabled() &&
+        plain_call({&rows, &rstd, &mean, w ? &*w : nullptr, b ? &*b : nullptr, &gy, &gh});
+    std::optional<at::AutoDispatchBelowADInplaceOrView> below;
+    if (direct) below.emplace();
+    if (!gy.defined()) gy = at::zeros_like(rows);
+    const Tensor x2 = as_rows(rows, n), dy2 = as_rows(gy.contiguous(), n);
+    const OptT extra = gh.defined() ? OptT(as_rows(gh.contiguous(), n)) : std::nullopt;
+    const OptT w1 = as_param(w), b1 = as_param(b);
+    Tensor dx, dw, db;
+    if (rms) {
+      std::tie(dx, dw) =
+          call(direct, "fused_layernorm::rms_norm_bwd", &rms_norm_bwd, dy2, x2, rstd, w1,
+               std::array<bool, 2>{need_x, need_w}, extra);
+    } else if (kind == kLayerNormGelu) {
+      std::tie(dx, dw, db) =
+          call(direct, "fused_layernorm::layer_norm_gelu_bwd", &layer_norm_gelu_bwd, dy2, x2,
+               mean, rstd, w1, b1, approximate, std::array<bool, 3>{need_x, need_w, need_b});
+    } else {
+      std::tie(dx, dw, db) =
+          call(direct, "fused_layernorm::layer_norm_bwd", &layer_norm_bwd, dy2, x2, mean, rstd,
+               w1, b1, std::array<bool, 3>{need_x, need_w, need_b}, extra);
+    }
+    if (need_x) {
+      if (dx.sizes() != rows.sizes()) dx = dx.view(rows.sizes());
+      if (task_should_compute_output(0)) out[0] = dx;
+      if (add && task_should_compute_output(1)) out[1] = dx;
+    }
+    if (need_w) out[2] = w->dim() == 1 ? dw : dw.view(w->sizes());
+    if (need_b) out[3] = b->dim() == 1 ? db : db.view(b->sizes());
+    return out;
+  }
+  std::string name() const override { return "FusedNormBackward"; }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    rows_.reset_data();
+    w_.reset_data();
+    b_.reset_data();
+    mean_.reset_data();
+    rstd_.reset_data();
+  }
+};
+
+// y, or (y, h) with a residual; nothing where the call has to go through the operators (or is not
+// valid: they raise the error).  input: [..., trailing dimensions of n elements].
+std::optional<std::vector<Tensor>> norm_autograd(int kind_code, const Tensor& input,
+                                                 const OptT& residual, int64_t n,
+                                                 const OptT& weight, const OptT& bias, double eps,
+                                                 const std::string& approximate) {
+  const NormKind kind = static_cast<NormKind>(kind_code);
+  const bool add = kind == kAddLayerNorm || kind == kAddRmsNorm;
+  const bool rms = kind == kRmsNorm || kind == kAddRmsNorm;
+  const Tensor none;
+  const Tensor& w = has(weight) ? *weight : none;
+  const Tensor& b = has(bias) && !rms ? *bias : none;
+  const Tensor& r = add && has(residual) ? *residual : none;
+  if (!input.defined() || n <= 0 || input.numel() % n != 0 || add != r.defined() ||
+      !plain_call({&input, &r, &w, &b}))
+    return std::nullopt;
+  const int code = dtype_code(input);
+  if (code < 0 || (rms && code == FLN_F64)) return std::nullopt;
+  for (const Tensor* p : {&w, &b})
+    if (p->defined() && (p->numel() != n || p->scalar_type() != input.scalar_type() ||
+                         p->device() != input.device()))
+      return std::nullopt;
+  if (add && (r.sizes() != input.sizes() || r.scalar_type() != input.scalar_type() ||
+              r.device() != input.device()))
+    return std::nullopt;
+  const Tensor x = input.contiguous(), res = add ? r.contiguous() : none;
+  Tensor y, h, mean, rstd;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor x2 = as_rows(x, n);
+    const OptT w1 = as_param(w.defined() ? OptT(w) : std::nullopt);
+    const OptT b1 = as_param(b.defined() ? OptT(b) : std::nullopt);
+    if ((w1 && !w1->is_contiguous()) || (b1 && !b1->is_contiguous())) return std::nullopt;
+    switch (kind) {
+      case kLayerNorm: std::tie(y, mean, rstd) = layer_norm_fwd(x2, w1, b1, eps); break;
+      case kRmsNorm: std::tie(y, rstd) = rms_norm_fwd(x2, w1, eps); break;
+      case kLayerNormGelu:
+        std::tie(y, mean, rstd) = layer_norm_gelu_fwd(x2, w1, b1, eps, approximate);
+        break;
+      case kAddLayerNorm:
+        std::tie(y, h, mean, rstd) = add_layer_norm_fwd(x2, as_rows(res, n), w1, b1, eps);
+        break;
+      case kAddRmsNorm: std::tie(y, h, rstd) = add_rms_norm_fwd(x2, as_rows(res, n), w1, eps); break;
+      default: return std::nullopt;
+    }
+    if (y.sizes() != x.sizes()) {
+      y = y.view(x.sizes());
+      if (add) h = h.view(x.sizes());
+    }
+  }
+  auto wants = [](const Tensor& t) { return t.defined() && t.requires_grad(); };
+  if (c10::GradMode::is_enabled() && (wants(x) || wants(res) || wants(w) || wants(b))) {
+    std::shared_ptr<FusedNormBackward> node(new FusedNormBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(x, res, w, b));
+    node->kind = kind;
+    node->n = n;
+    node->approximate = approximate;
+    node->has_w = w.defined();
+    node->has_b = b.defined();
+    torch::autograd::set_history(y, node);
+    if (add) torch::autograd::set_history(h, node);
+    node->rows_ = torch::autograd::SavedVariable(add ? h : x, add);
+    if (node->has_w) node->w_ = torch::autograd::SavedVariable(w, false);
+    if (node->has_b) node->b_ = torch::autograd::SavedVariable(b, false);
+    if (!rms) node->mean_ = torch::autograd::SavedVariable(mean, false);
+    node->rstd_ = torch::autograd::SavedVariable(rstd, false);
+  }
+  if (add) return std::vector<Tensor>{y, h};
+  return std::vector<Tensor>{y};
+}
+
+// The quantized forwards of ordinary tensors of which autograd records nothing: the functions the
+// operators call, without the operators' dispatch and the views around it (residual add + RMSNorm
+// -> MXFP8 of 64 x 7168, host-bound, 15.9 -> 7.0 us).
+std::optional<std::vector<Tensor>> norm_quantized(int kind_code, bool mx, const Tensor& input,
+                                                  const OptT& residual, int64_t trailing,
+                                                  int64_t n, const OptT& weight, const OptT& bias,
+                                                  double eps) {
+  const NormKind kind = static_cast<NormKind>(kind_code);
+  const bool add = kind == kAddLayerNorm || kind == kAddRmsNorm;
+  const Tensor none;
+  const Tensor& w = has(weight) ? *weight : none;
+  const Tensor& b = has(bias) ? *bias : none;
+  const Tensor& r = add && has(residual) ? *residual : none;
+  if (!input.defined() || n <= 0 || input.numel() == 0 || input.numel() % n != 0 ||
+      trailing < 1 || trailing > input.dim() || add != r.defined() ||
+      !plain_call({&input, &r, &w, &b}))
+    return std::nullopt;
+  if (add && r.sizes() != input.sizes()) return std::nullopt;
+  if (c10::GradMode::is_enabled())
+    for (const Tensor* t : {&input, &r, &w, &b})
+      if (t->defined() && t->requires_grad()) return std::nullopt;
+  at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor x = as_rows(input.contiguous(), n), res = add ? as_rows(r.contiguous(), n) : none;
+  const OptT w1 = as_param(w.defined() ? OptT(w) : std::nullopt);
+  const OptT b1 = as_param(b.defined() ? OptT(b) : std::nullopt);
+  Tensor q, sc, h;
+  if (mx) {
+    switch (kind) {
+      case kLayerNorm: std::tie(q, sc) = layer_norm_mxfp8_fwd(x, w1, b1, eps); break;
+      case kRmsNorm: std::tie(q, sc) = rms_norm_mxfp8_fwd(x, w1, eps); break;
+      case kAddRmsNorm: std::tie(q, sc, h) = add_rms_norm_mxfp8_fwd(x, res, w1, eps); break;
+      default: return std::nullopt;
+    }
+  } else {
+    switch (kind) {
+      case kLayerNorm: std::tie(q, sc) = layer_norm_fp8_fwd(x, w1, b1, eps); break;
+      case kRmsNorm: std::tie(q, sc) = rms_norm_fp8_fwd(x, w1, eps); break;
+      case kAddLayerNorm: std::tie(q, sc, h) = add_layer_norm_fp8_fwd(x, res, w1, b1, eps); break;
+      case kAddRmsNorm: std::tie(q, sc, h) = add_rms_norm_fp8_fwd(x, res, w1, eps); break;
+      default: return std::nullopt;
+    }
+  }
+  if (q.sizes() != input.sizes()) {
+    q = q.view(input.sizes());
+    if (add) h = h.view(input.sizes());
+  }
+  if (trailing != 1 || input.dim() != 2) {
+    std::vector<int64_t> shape(input.sizes().begin(), input.sizes().end() - trailing);
+    if (mx)
+      shape.push_back(n / 32);
+    else if (shape.empty())
+      shape.push_back(1);
+    sc = sc.view(shape);
+  }
+  if (add) return std::vector<Tensor>{q, sc, h};
+  return std::vector<Tensor>{q, sc};
+}
+
 // The forward launch plan (fln_forward_plan): (route, vector_elems, waves_per_row,
 // vectors_per_lane, exact, threads) for a contiguous, aligned input; backs
 // fused_layernorm.functional.get_optimal_config (reference fused_layernorm/functional.py:47-74).
@@ -812,6 +1060,19 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "RMSNorm over the last dimension with autograd in C++ (FusedRMSNorm's eager path)",
         py::arg("input"), py::arg("normalized"), py::arg("weight") = py::none(),
         py::arg("eps") = 1e-6);
+  m.def("norm_autograd", &norm_autograd,
+        "Eager differentiable norms with autograd in C++ (kind 0 LayerNorm, 1 RMSNorm, 2 LayerNorm "
+        "+ GELU, 3 residual add + LayerNorm, 4 residual add + RMSNorm) over trailing dimensions of "
+        "n elements -> [y] or [y, h], or None where the operators have to be used",
+        py::arg("kind"), py::arg("input"), py::arg("residual"), py::arg("n"), py::arg("weight"),
+        py::arg("bias"), py::arg("eps"), py::arg("approximate") = "tanh");
+  m.def("norm_quantized", &norm_quantized,
+        "Eager quantized norms of which autograd records nothing (kind 0 LayerNorm, 1 RMSNorm, 3 "
+        "residual add + LayerNorm, 4 residual add + RMSNorm; mx: OCP MX block scales) over the last "
+        "`trailing` dimensions -> [codes, scales] or [codes, scales, h], or None where the "
+        "operators have to be used",
+        py::arg("kind"), py::arg("mx"), py::arg("input"), py::arg("residual"),
+        py::arg("trailing"), py::arg("n"), py::arg("weight"), py::arg("bias"), py::arg("eps"));
   m.def("forward_plan", &forward_plan,
         "Forward launch plan -> (route, vector_elems, waves_per_row, vectors_per_lane, exact, "
         "threads); dtype / gelu are the C-ABI codes, num_cus 0 = the current device",

@@ -89,6 +89,9 @@ def _apply_rows(input: torch.Tensor, normalized_shape: Tuple[int, ...],
             f"Given normalized_shape={list(normalized_shape)}, expected input with shape "
             f"[*, {', '.join(str(s) for s in normalized_shape)}], but got input of size "
             f"{list(input.shape)}")
+    out = _fops._eager_norm(_fops._LN, input, None, normalized_shape, weight, bias, eps)
+    if out is not None:
+        return out[0]
     n = math.prod(normalized_shape)
     x2 = input.reshape(-1, n)
     w = None if weight is None else weight.reshape(-1)

@@ -295,10 +295,56 @@ def _flat_param(p: Optional[torch.Tensor]):
     return None if p is None else p.reshape(-1)
 
 
+# The eager paths below pass the operators by where nothing can tell the difference: ordinary
+# tensors outside torch.compile, with no __torch_function__ mode; the extension refuses the rest
+# (dispatch modes, tracing, functorch transforms, forward-mode tangents).
+_ORDINARY = (torch.Tensor, torch.nn.Parameter)
+_compiling = torch.compiler.is_compiling
+_function_modes = torch._C._len_torch_function_stack
+_LN, _RMS, _LN_GELU, _ADD_LN, _ADD_RMS = range(5)  # _ext.norm_autograd's kinds
+
+
+def _ordinary(*tensors: Optional[torch.Tensor]) -> bool:
+    if _compiling() or _function_modes():
+        return False
+    for t in tensors:
+        if t is not None and type(t) not in _ORDINARY:
+            return False
+    return True
+
+
+def _eager_norm(kind: int, input: torch.Tensor, residual: Optional[torch.Tensor],
+                normalized_shape: ShapeLike, weight: Optional[torch.Tensor],
+                bias: Optional[torch.Tensor], eps: float, approximate: str = "tanh"):
+    """The call with autograd in C++ -> [y] or [y, h], or None: through the operators."""
+    if not _ordinary(input, residual, weight, bias):
+        return None
+    ns = _norm_shape(normalized_shape)
+    if not ns or input.shape[-len(ns):] != ns:
+        return None
+    return _ext.norm_autograd(kind, input, residual, math.prod(ns), weight, bias, eps, approximate)
+
+
+def _eager_quantized(kind: int, mx: bool, input: torch.Tensor,
+                     residual: Optional[torch.Tensor], normalized_shape: ShapeLike,
+                     weight: Optional[torch.Tensor], bias: Optional[torch.Tensor], eps: float):
+    """The quantized forward without the operators -> its outputs, or None: through them (as where
+    a gradient is recorded)."""
+    if not _ordinary(input, residual, weight, bias):
+        return None
+    ns = _norm_shape(normalized_shape)
+    if not ns or input.shape[-len(ns):] != ns:
+        return None
+    return _ext.norm_quantized(kind, mx, input, residual, len(ns), math.prod(ns), weight, bias, eps)
+
+
 def layer_norm(input: torch.Tensor, normalized_shape: ShapeLike,
                weight: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
                eps: float = 1e-5) -> torch.Tensor:
     """LayerNorm with torch.nn.functional.layer_norm semantics (weight / bias independent)."""
+    out = _eager_norm(_LN, input, None, normalized_shape, weight, bias, eps)
+    if out is not None:
+        return out[0]
     x, _ = _flatten(input, normalized_shape)
     y, _, _ = _ops.layer_norm_fwd(x, _flat_param(weight), _flat_param(bias), eps)
     return y.view(input.shape)
@@ -310,6 +356,9 @@ def layer_norm_gelu(input: torch.Tensor, normalized_shape: ShapeLike,
     """GELU(LayerNorm(x)); approximate='tanh' is the reference's fused GELU, 'none' the exact
     erf form.  Differentiable: the backward recomputes the GELU input from the saved row
     statistics and folds GELU' into the fused LayerNorm backward."""
+    out = _eager_norm(_LN_GELU, input, None, normalized_shape, weight, bias, eps, approximate)
+    if out is not None:
+        return out[0]
     x, _ = _flatten(input, normalized_shape)
     y, _, _ = _ops.layer_norm_gelu_fwd(x, _flat_param(weight), _flat_param(bias), eps,
                                        approximate)
@@ -325,6 +374,9 @@ def rms_norm(input: torch.Tensor, normalized_shape: ShapeLike,
     if len(ns) == 1 and not torch.compiler.is_compiling():
         # Eager: autograd in C++ around the kernels (FusedRMSNorm's hot path).
         return _ext.rms_norm_autograd(input, ns[0], weight, eps)
+    out = _eager_norm(_RMS, input, None, ns, weight, None, eps)
+    if out is not None:
+        return out[0]
     x, _ = _flatten(input, normalized_shape)
     y, _ = _ops.rms_norm_fwd(x, _flat_param(weight), eps)
     return y.view(input.shape)
@@ -334,6 +386,9 @@ def add_layer_norm(input: torch.Tensor, residual: torch.Tensor, normalized_shape
                    weight: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
                    eps: float = 1e-5) -> Tuple[torch.Tensor, torch.Tensor]:
     """Fused residual add + LayerNorm -> (LayerNorm(h), h) with h = input + residual."""
+    out = _eager_norm(_ADD_LN, input, residual, normalized_shape, weight, bias, eps)
+    if out is not None:
+        return out[0], out[1]
     x, _ = _flatten(input, normalized_shape)
     r, _ = _flatten(residual, normalized_shape)
     y, h, _, _ = _ops.add_layer_norm_fwd(x, r, _flat_param(weight), _flat_param(bias), eps)
@@ -344,6 +399,9 @@ def add_rms_norm(input: torch.Tensor, residual: torch.Tensor, normalized_shape: 
                  weight: Optional[torch.Tensor] = None, eps: float = 1e-6
                  ) -> Tuple[torch.Tensor, torch.Tensor]:
     """Fused residual add + RMSNorm -> (RMSNorm(h), h) with h = input + residual."""
+    out = _eager_norm(_ADD_RMS, input, residual, normalized_shape, weight, None, eps)
+    if out is not None:
+        return out[0], out[1]
     x, _ = _flatten(input, normalized_shape)
     r, _ = _flatten(residual, normalized_shape)
     y, h, _ = _ops.add_rms_norm_fwd(x, r, _flat_param(weight), eps)
@@ -355,6 +413,9 @@ def layer_norm_fp8(input: torch.Tensor, normalized_shape: ShapeLike,
                    eps: float = 1e-5) -> Tuple[torch.Tensor, torch.Tensor]:
     """LayerNorm quantized to OCP fp8 e4m3fn -> (codes as torch.float8_e4m3fn, per-row float32
     scale); dequantize with codes.float() * scale[..., None]."""
+    out = _eager_quantized(_LN, False, input, None, normalized_shape, weight, bias, eps)
+    if out is not None:
+        return tuple(out)
     x, _ = _flatten(input, normalized_shape)
     q, scale = _ops.layer_norm_fp8_fwd(x, _flat_param(weight), _flat_param(bias), eps)
     lead = tuple(input.shape[:input.dim() - len(_norm_shape(normalized_shape))])
@@ -365,6 +426,9 @@ def rms_norm_fp8(input: torch.Tensor, normalized_shape: ShapeLike,
                  weight: Optional[torch.Tensor] = None, eps: float = 1e-6
                  ) -> Tuple[torch.Tensor, torch.Tensor]:
     """RMSNorm quantized to OCP fp8 e4m3fn -> (codes, per-row float32 scale)."""
+    out = _eager_quantized(_RMS, False, input, None, normalized_shape, weight, None, eps)
+    if out is not None:
+        return tuple(out)
     x, _ = _flatten(input, normalized_shape)
     q, scale = _ops.rms_norm_fp8_fwd(x, _flat_param(weight), eps)
     lead = tuple(input.shape[:input.dim() - len(_norm_shape(normalized_shape))])
@@ -376,6 +440,9 @@ def add_layer_norm_fp8(input: torch.Tensor, residual: torch.Tensor, normalized_s
                        eps: float = 1e-5) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Fused residual add + LayerNorm -> fp8: (codes, per-row scale, h = input + residual).
     Gradients flow through h only (to input and residual)."""
+    out = _eager_quantized(_ADD_LN, False, input, residual, normalized_shape, weight, bias, eps)
+    if out is not None:
+        return tuple(out)
     x, _ = _flatten(input, normalized_shape)
     r, _ = _flatten(residual, normalized_shape)
     q, scale, h = _ops.add_layer_norm_fp8_fwd(x, r, _flat_param(weight), _flat_param(bias), eps)
@@ -388,6 +455,9 @@ def add_rms_norm_fp8(input: torch.Tensor, residual: torch.Tensor, normalized_sha
                      ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Fused residual add + RMSNorm -> fp8 (the pre-norm feeding an fp8 GEMM):
     (codes, per-row scale, h = input + residual).  Gradients flow through h only."""
+    out = _eager_quantized(_ADD_RMS, False, input, residual, normalized_shape, weight, None, eps)
+    if out is not None:
+        return tuple(out)
     x, _ = _flatten(input, normalized_shape)
     r, _ = _flatten(residual, normalized_shape)
     q, scale, h = _ops.add_rms_norm_fp8_fwd(x, r, _flat_param(weight), eps)
@@ -400,6 +470,9 @@ def layer_norm_mxfp8(input: torch.Tensor, normalized_shape: ShapeLike,
                      eps: float = 1e-5) -> Tuple[torch.Tensor, torch.Tensor]:
     """LayerNorm quantized to OCP MXFP8 E4M3 -> (codes float8_e4m3fn, E8M0 block scales
     float8_e8m0fnu [..., n / 32]); dequantize block-wise with codes.float() * scales.float()."""
+    out = _eager_quantized(_LN, True, input, None, normalized_shape, weight, bias, eps)
+    if out is not None:
+        return tuple(out)
     x, n = _flatten(input, normalized_shape)
     q, sc = _ops.layer_norm_mxfp8_fwd(x, _flat_param(weight), _flat_param(bias), eps)
     lead = tuple(input.shape[:input.dim() - len(_norm_shape(normalized_shape))])
@@ -410,6 +483,9 @@ def rms_norm_mxfp8(input: torch.Tensor, normalized_shape: ShapeLike,
                    weight: Optional[torch.Tensor] = None, eps: float = 1e-6
                    ) -> Tuple[torch.Tensor, torch.Tensor]:
     """RMSNorm quantized to OCP MXFP8 E4M3 -> (codes, E8M0 block scales)."""
+    out = _eager_quantized(_RMS, True, input, None, normalized_shape, weight, None, eps)
+    if out is not None:
+        return tuple(out)
     x, n = _flatten(input, normalized_shape)
     q, sc = _ops.rms_norm_mxfp8_fwd(x, _flat_param(weight), eps)
     lead = tuple(input.shape[:input.dim() - len(_norm_shape(normalized_shape))])
@@ -421,6 +497,9 @@ def add_rms_norm_mxfp8(input: torch.Tensor, residual: torch.Tensor, normalized_s
                        ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Fused residual add + RMSNorm -> OCP MXFP8 E4M3: (codes, E8M0 block scales,
     h = input + residual).  Gradients flow through h only."""
+    out = _eager_quantized(_ADD_RMS, True, input, residual, normalized_shape, weight, None, eps)
+    if out is not None:
+        return tuple(out)
     x, n = _flatten(input, normalized_shape)
     r, _ = _flatten(residual, normalized_shape)
     q, sc, h = _ops.add_rms_norm_mxfp8_fwd(x, r, _flat_param(weight), eps)
