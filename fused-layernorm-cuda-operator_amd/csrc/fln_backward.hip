@@ -837,7 +837,8 @@ __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdPara
   }
 }
 
-template <class T, bool DRES, int GELU, int VEC, bool RAGGED>
+// OWN (ragged rows with dx over an input): the row's last vector is written by element.
+template <class T, bool DRES, int GELU, int VEC, bool RAGGED, bool OWN = false>
 __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdParams p,
                                                                    const float2* stats) {
   using P = Pack<T, VEC>;
@@ -847,6 +848,9 @@ __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdPara
   const int nvec = RAGGED ? static_cast<int>(rag.nvec) : static_cast<int>(N / VEC);
   const uint32_t off = RAGGED ? rag.off(static_cast<uint32_t>(v))
                               : static_cast<uint32_t>(v) * static_cast<uint32_t>(sizeof(P));
+  // OWN: the block that holds the row's last vector writes only that vector's own elements.
+  const bool tail = OWN && (blockIdx.x + 1) * kWideThreads > rag.nfull;  // uniform
+  const int lo = OWN ? rag.lo(static_cast<uint32_t>(v)) : 0;
   const uint32_t row_bytes = static_cast<uint32_t>(N * sizeof(T));
   const float inv_n = 1.0f / static_cast<float>(N);
   // Block y takes rows y, y + G, y + 2G, ... (G = gridDim.y): all blocks stream through one
@@ -910,17 +914,20 @@ __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdPara
           acc_b[e] += d;
         }
       }
-      buf_store_at<P, kStream>(o, make_rsrc(DX ? DX + r * N : nullptr, in ? row_bytes : 0u), off);
+      const rsrc_t xo = make_rsrc(DX ? DX + r * N : nullptr, in ? row_bytes : 0u);
+      if (tail)
+        buf_store_own<T, VEC, kStream>(o, xo, off, lo);
+      else
+        buf_store_at<P, kStream>(o, xo, off);
     }
   }
   if (v >= nvec) return;
-  // (A ragged row's last vector writes the columns it shares with the vector before it as well:
-  // the same sums.)
   const int64_t col = RAGGED ? static_cast<int64_t>(off / static_cast<uint32_t>(sizeof(T)))
                              : static_cast<int64_t>(v) * VEC;
   if (p.out_g != nullptr || p.out_b != nullptr) {  // one block row: these sums are final
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
+      if (OWN && e < lo) continue;
       const int64_t j = col + e;
       if (p.out_g) store_param(p.out_g, p.out_dtype, j, acc_g[e]);
       if (p.out_b) store_param(p.out_b, p.out_dtype, j, acc_b[e]);
@@ -930,12 +937,15 @@ __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdPara
   const int64_t ld = (N + 3) & ~int64_t(3);
   const int64_t c = static_cast<int64_t>(blockIdx.y) * ld + col;
   if constexpr (RAGGED) {
-    if (p.part_g) store_columns<VEC>(p.part_g + c, acc_g);
-    if (p.part_b) store_columns<VEC>(p.part_b + c, acc_b);
-    return;
+    if (lo == 0) {
+      if (p.part_g) store_columns<VEC>(p.part_g + c, acc_g);
+      if (p.part_b) store_columns<VEC>(p.part_b + c, acc_b);
+      return;
+    }
   }
 #pragma unroll
   for (int e = 0; e < VEC; ++e) {
+    if (OWN && e < lo) continue;
     if (p.part_g) p.part_g[c + e] = acc_g[e];
     if (p.part_b) p.part_b[c + e] = acc_b[e];
   }
@@ -1198,6 +1208,28 @@ int launch_two_pass(const BwdParams& p, const BwdGeometry& geo, hipStream_t s) {
   const int64_t nvec = (p.cols + VEC - 1) / VEC;
   const dim3 g2(static_cast<unsigned>((nvec + kWideThreads - 1) / kWideThreads),
                 static_cast<unsigned>(geo.blocks));
+  if constexpr (RAGGED) {
+    const int64_t bytes = p.rows * p.cols * static_cast<int64_t>(sizeof(T));
+    if (overlaps(p.dx, bytes, p.x, bytes) || overlaps(p.dx, bytes, p.dy, bytes) ||
+        overlaps(p.dx, bytes, p.dres, bytes)) {
+      auto run = [&](auto rowstat, auto colpass) {
+        hipLaunchKernelGGL(rowstat, g1, blk, 0, s, p, stats);
+        hipLaunchKernelGGL(colpass, g2, blk, 0, s, p, stats);
+        return static_cast<int>(hipGetLastError());
+      };
+      if (p.gelu == 1)
+        return run(bwd_rowstat_kernel<T, 1, VEC, true>,
+                   bwd_colpass_kernel<T, false, 1, VEC, true, true>);
+      if (p.gelu == 2)
+        return run(bwd_rowstat_kernel<T, 2, VEC, true>,
+                   bwd_colpass_kernel<T, false, 2, VEC, true, true>);
+      if (p.dres)
+        return run(bwd_rowstat_kernel<T, 0, VEC, true>,
+                   bwd_colpass_kernel<T, true, 0, VEC, true, true>);
+      return run(bwd_rowstat_kernel<T, 0, VEC, true>,
+                 bwd_colpass_kernel<T, false, 0, VEC, true, true>);
+    }
+  }
   if (p.gelu == 1) {
     hipLaunchKernelGGL((bwd_rowstat_kernel<T, 1, VEC, RAGGED>), g1, blk, 0, s, p, stats);
     hipLaunchKernelGGL((bwd_colpass_kernel<T, false, 1, VEC, RAGGED>), g2, blk, 0, s, p, stats);

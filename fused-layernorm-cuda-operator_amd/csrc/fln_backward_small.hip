@@ -1,0 +1,337 @@
+// fln_backward_small.hip -- the backward of small problems in one launch, without a workspace.
+//
+// With few rows the two-stage backward is bound by latency: stage 1, the hand-over of its partial
+// rows through memory, a second launch to sum them, and, for rows past the register tiles, a third
+// for their statistics.  dx needs sums over a row and dgamma / dbeta sums over the columns, but
+// neither needs the other, and a small x and dy are served from L2 the second time.  So the blocks
+// of one launch take two roles:
+//   dx blocks (the first p.dx_blocks): whole rows, each in the registers of `wpr` waves, up to 8
+//     vectors per lane in the I/O type (65536 16-bit or 32768 fp32 columns: without column sums to
+//     carry, a 1024-thread block holds x and dy of a row that wide); as bwd_reg_kernel otherwise.
+//   column blocks: 64 vector columns each, one per lane, over every row: 16 waves take every 16th
+//     row with 8 in flight, then the 16 partial sums of a column are added in order through LDS.
+// Both roles take unaligned vectors (RaggedRow), so any width of at least one vector runs here.
+#include <type_traits>
+
+#include "fln_device.h"
+#include "fln_internal.h"
+
+namespace fln {
+namespace {
+
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / kWave;
+
+struct SmallArgs {
+  BwdParams p;
+  int dx_blocks;  // blocks of the dx role (0: dx not requested)
+  int groups;     // row groups per dx block
+};
+
+template <class T, bool DRES, int GELU, int VEC, int VPL>
+__global__ __launch_bounds__(kSmallThreads) void bwd_small_kernel(const SmallArgs a) {
+  using P = Pack<T, VEC>;
+  const BwdParams& p = a.p;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t N = p.cols;
+  const uint32_t row_bytes = static_cast<uint32_t>(N * sizeof(T));
+  const RaggedRow<T, VEC> rag(static_cast<uint32_t>(N));
+  const T* X = static_cast<const T*>(p.x);
+  const T* DY = static_cast<const T*>(p.dy);
+  const rsrc_t g_rs = make_rsrc(p.gamma, row_bytes);
+  const rsrc_t b_rs = make_rsrc(p.beta, row_bytes);  // GELU only; absent beta reads as zeros
+  const bool has_g = p.gamma != nullptr;
+  __shared__ float4 gelu_tab[GELU != 0 ? kGeluTabN : 1];
+  if constexpr (GELU != 0) {
+    if (threadIdx.x < kGeluTabN)
+      gelu_tab[threadIdx.x] = reinterpret_cast<const float4*>(
+          GELU == 1 ? kGeluTabData : kGeluTanhTabData)[threadIdx.x];
+  }
+  // Gradient at the LayerNorm output of one element: dy, or dy GELU'(xhat gamma + beta).
+  auto upstream = [&](float d, float xh, float g, float b) -> float {
+    if constexpr (GELU != 0) {
+      const float u = kGeluTabInvH * fmaf(xh, g, b);
+      d = 0.5f * fmaf(d, gelu_grad2_sign_tab(gelu_tab, u), d);
+    }
+    (void)xh, (void)g, (void)b;
+    return d;
+  };
+
+  if (static_cast<int>(blockIdx.x) < a.dx_blocks) {
+    __shared__ float red[2][kSmallWaves + 16];  // padded for combine_partials
+    const int wpr = p.wpr;
+    const int rg = wave / wpr;
+    const int t = (wave - rg * wpr) * kWave + lane;
+    const int tpr = kWave * wpr;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * a.groups + rg;
+    const bool in = rg < a.groups && row < p.rows;
+    const uint32_t nb = in ? row_bytes : 0u;  // no row: reads zeros, stores nothing
+    const int64_t r = in ? row : 0;
+    // Up to 2 vectors per lane gamma, beta and the residual gradient are loaded with the row; wider
+    // tiles have no registers for them and read them where they are used.
+    constexpr bool PRELOAD = VPL <= 2;
+    const rsrc_t xr = make_rsrc(X + r * N, nb), dr = make_rsrc(DY + r * N, nb);
+    const rsrc_t rr = make_rsrc(DRES ? static_cast<const T*>(p.dres) + r * N : nullptr, nb);
+    uint32_t off[VPL];
+    P xv[VPL], dv[VPL], gp[PRELOAD ? VPL : 1], bp[PRELOAD && GELU ? VPL : 1],
+        rp[PRELOAD && DRES ? VPL : 1];
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      off[i] = rag.off(static_cast<uint32_t>(t + i * tpr));
+      xv[i] = buf_load_at<P>(xr, off[i]);
+      dv[i] = buf_load_at<P>(dr, off[i]);
+      if constexpr (PRELOAD) {
+        gp[i] = buf_load_at<P>(g_rs, off[i]);
+        if constexpr (GELU != 0) bp[i] = buf_load_at<P>(b_rs, off[i]);
+        if constexpr (DRES) rp[i] = buf_load_at<P>(rr, off[i]);
+      }
+    }
+    const uint32_t sb = in ? 4u : 0u;
+    const float mu = __builtin_bit_cast(
+        float, BufIO<4>::load(make_rsrc(p.rms ? nullptr : p.mean + r, sb), 0));
+    const float rs = __builtin_bit_cast(float, BufIO<4>::load(make_rsrc(p.rstd + r, sb), 0));
+    if constexpr (GELU != 0) __syncthreads();  // the table
+    auto gamma = [&](int i) -> P {
+      if constexpr (PRELOAD)
+        return gp[i];
+      else
+        return buf_load_at<P>(g_rs, off[i]);
+    };
+    auto beta = [&](int i) -> P {
+      if constexpr (GELU == 0)
+        return P{};
+      else if constexpr (PRELOAD)
+        return bp[i];
+      else
+        return buf_load_at<P>(b_rs, off[i]);
+    };
+    float s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const P gv = gamma(i), bv = beta(i);
+      const int lo = rag.lo(static_cast<uint32_t>(t + i * tpr));
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const float xh = (to_f32(xv[i].v[e]) - mu) * rs;
+        const float gm = has_g ? to_f32(gv.v[e]) : 1.0f;
+        const float g = upstream(to_f32(dv[i].v[e]), xh, gm, GELU ? to_f32(bv.v[e]) : 0.0f) * gm;
+        if (e >= lo) {  // the last vector's own elements
+          s1 += g;
+          s2 = fmaf(g, xh, s2);
+        }
+      }
+    }
+    s1 = wave_allreduce<SumOp>(s1);
+    s2 = wave_allreduce<SumOp>(s2);
+    if (wpr > 1) {
+      if (lane == 0) {
+        red[0][wave] = s1;
+        red[1][wave] = s2;
+      }
+      __syncthreads();
+      s1 = combine_partials<SumOp>(red[0], rg * wpr, wpr, lane, 0.0f);
+      s2 = combine_partials<SumOp>(red[1], rg * wpr, wpr, lane, 0.0f);
+    }
+    const float inv_n = 1.0f / static_cast<float>(N);
+    const float cb = p.rms ? 0.0f : -rs * (s1 * inv_n);
+    const float cx = -rs * (s2 * inv_n);
+    const rsrc_t xo = make_rsrc(static_cast<T*>(p.dx) + r * N, nb);
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      if constexpr (!PRELOAD) {  // widened again from the packs, not kept in fp32 across the sums
+        keep_packed(xv[i]);
+        keep_packed(dv[i]);
+      }
+      const P gv = gamma(i), bv = beta(i);
+      P rv{};
+      if constexpr (DRES) {
+        if constexpr (PRELOAD)
+          rv = rp[i];
+        else
+          rv = buf_load_at<P>(rr, off[i]);
+      }
+      P o;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const float xh = (to_f32(xv[i].v[e]) - mu) * rs;
+        const float gm = has_g ? to_f32(gv.v[e]) : 1.0f;
+        const float d = upstream(to_f32(dv[i].v[e]), xh, gm, GELU ? to_f32(bv.v[e]) : 0.0f);
+        float dxv = fmaf(rs, d * gm, fmaf(cx, xh, cb));
+        if constexpr (DRES) dxv += to_f32(rv.v[e]);
+        o.v[e] = from_f32<T>(dxv);
+      }
+      buf_store_at<P>(o, xo, off[i]);
+    }
+    return;
+  }
+
+  // Column role.  Rows in flight per wave: 8 (4 with GELU on 8 columns, which spilled).
+  constexpr int kColUnroll = GELU != 0 && VEC == 8 ? 4 : 8;
+  constexpr int kCols = kWave * VEC;  // columns of a block
+  __shared__ float part[2][kSmallWaves][kCols];
+  const uint32_t v0 = (blockIdx.x - static_cast<uint32_t>(a.dx_blocks)) * kWave;
+  const uint32_t off = rag.off(v0 + lane);
+  const P gv = buf_load_at<P>(g_rs, off);
+  P bv{};
+  if constexpr (GELU != 0) {
+    bv = buf_load_at<P>(b_rs, off);
+    __syncthreads();  // the table
+  }
+  float acc_g[VEC], acc_b[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) acc_g[e] = acc_b[e] = 0.0f;
+  for (int64_t row = wave; row < p.rows; row += kColUnroll * kSmallWaves) {
+    P xv[kColUnroll], dv[kColUnroll];
+    float mu[kColUnroll], rs[kColUnroll];
+#pragma unroll
+    for (int u = 0; u < kColUnroll; ++u) {
+      // Rows past the tensor read as zeros, statistics included: they add exact zeros.
+      const bool in = row + u * kSmallWaves < p.rows;  // uniform
+      const int64_t r = in ? row + u * kSmallWaves : row;
+      const uint32_t nb = in ? row_bytes : 0u, sb = in ? 4u : 0u;
+      xv[u] = buf_load_at<P>(make_rsrc(X + r * N, nb), off);
+      dv[u] = buf_load_at<P>(make_rsrc(DY + r * N, nb), off);
+      mu[u] = __builtin_bit_cast(
+          float, BufIO<4>::load(make_rsrc(p.rms ? nullptr : p.mean + r, sb), 0));
+      rs[u] = __builtin_bit_cast(float, BufIO<4>::load(make_rsrc(p.rstd + r, sb), 0));
+    }
+#pragma unroll
+    for (int u = 0; u < kColUnroll; ++u)
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const float xh = (to_f32(xv[u].v[e]) - mu[u]) * rs[u];
+        const float d = upstream(to_f32(dv[u].v[e]), xh, has_g ? to_f32(gv.v[e]) : 1.0f,
+                                 GELU ? to_f32(bv.v[e]) : 0.0f);
+        acc_g[e] = fmaf(d, xh, acc_g[e]);
+        acc_b[e] += d;
+      }
+  }
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    part[0][wave][lane * VEC + e] = acc_g[e];
+    part[1][wave][lane * VEC + e] = acc_b[e];
+  }
+  __syncthreads();
+  if (threadIdx.x >= 2 * kCols) return;
+  const int which = threadIdx.x / kCols, c = threadIdx.x % kCols;
+  const uint32_t v = v0 + static_cast<uint32_t>(c / VEC);
+  void* out = which == 0 ? p.out_g : p.out_b;
+  if (out == nullptr || c % VEC < rag.lo(v)) return;  // (lo = VEC past the row)
+  float s = part[which][0][c];
+#pragma unroll
+  for (int k = 1; k < kSmallWaves; ++k) s += part[which][k][c];
+  store_param(out, p.out_dtype, rag.off(v) / static_cast<uint32_t>(sizeof(T)) + c % VEC, s);
+}
+
+template <class T, int VPL>
+int launch_vpl(const SmallArgs& a, int blocks, hipStream_t s) {
+  constexpr int VEC = 16 / sizeof(T);
+  if (a.p.gelu == FLN_GELU_ERF) {
+    static std::atomic<void*> cache[64];
+    return launch_cached(bwd_small_kernel<T, false, 1, VEC, VPL>, cache, dim3(blocks),
+                         dim3(kSmallThreads), s, a);
+  }
+  if (a.p.gelu == FLN_GELU_TANH) {
+    static std::atomic<void*> cache[64];
+    return launch_cached(bwd_small_kernel<T, false, 2, VEC, VPL>, cache, dim3(blocks),
+                         dim3(kSmallThreads), s, a);
+  }
+  if (a.p.dres) {
+    static std::atomic<void*> cache[64];
+    return launch_cached(bwd_small_kernel<T, true, 0, VEC, VPL>, cache, dim3(blocks),
+                         dim3(kSmallThreads), s, a);
+  }
+  static std::atomic<void*> cache[64];
+  return launch_cached(bwd_small_kernel<T, false, 0, VEC, VPL>, cache, dim3(blocks),
+                       dim3(kSmallThreads), s, a);
+}
+
+struct SmallPlan {
+  int wpr, vpl, groups, dx_blocks, col_blocks;
+};
+
+// Waves per row (1..16) and vectors per lane (1, 2, 4 or 8) of the dx role; vpl 0: too wide.
+SmallPlan plan(const BwdParams& p, int es) {
+  SmallPlan s{};
+  const int64_t vec = 16 / es, nvec = (p.cols + vec - 1) / vec;
+  const int64_t cus = device_cu_count();
+  const int64_t slots = (nvec + kWave - 1) / kWave;  // wave-wide vectors of a row
+  s.vpl = slots <= 16 ? 1 : slots <= 32 ? 2 : slots <= 64 ? 4 : slots <= 128 ? 8 : 0;
+  if (s.vpl == 0) return s;
+  s.wpr = static_cast<int>((slots + s.vpl - 1) / s.vpl);
+  s.col_blocks = p.out_g || p.out_b ? static_cast<int>(slots) : 0;
+  if (p.dx) {
+    // One row per block while the blocks still fit the CUs, then as many as a block holds.
+    const int64_t room = cus > 2 * s.col_blocks ? cus - s.col_blocks : cus / 2;
+    int64_t groups = (p.rows + room - 1) / room;
+    const int most = kSmallWaves / s.wpr;
+    if (groups > most) groups = most;
+    s.groups = static_cast<int>(groups);
+    s.dx_blocks = static_cast<int>((p.rows + groups - 1) / groups);
+  }
+  return s;
+}
+
+// Byte ranges [a, a + na) and [b, b + nb) overlap (null pointers never do).
+bool overlaps(const void* a, int64_t na, const void* b, int64_t nb) {
+  if (a == nullptr || b == nullptr) return false;
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x < y + static_cast<uintptr_t>(nb) && y < x + static_cast<uintptr_t>(na);
+}
+
+}  // namespace
+
+bool backward_is_small(const BwdParams& p, const void* dgamma, const void* dbeta, int dtype) {
+  const Tuning& tun = tuning();
+  if (tun.bwd_small_rows < 0 || tun.bwd_epl > 0 || tun.bwd_wpr > 0 || tun.bwd_threads > 0 ||
+      tun.bwd_grid_mult > 0 || tun.bwd_no_lds || tun.bwd_no_two_pass || tun.bwd_stat_splits > 0 ||
+      tun.bwd_colpass_per_cu > 0)
+    return false;
+  const int es = element_size(dtype);
+  const int64_t vec = 16 / es;
+  if (p.cols < vec || p.cols > 16 * kWave * 8 * vec) return false;
+  const int64_t limit = tun.bwd_small_rows > 0 ? tun.bwd_small_rows : device_cu_count();
+  if (p.rows > limit) return false;
+  // The roles run at the same time: an output in place of an input (dx over dy, say) would be
+  // written while other blocks still read it.
+  const int64_t bytes = p.rows * p.cols * es, param = p.cols * es, stat = p.rows * 4;
+  const std::pair<const void*, int64_t> in[] = {{p.x, bytes},    {p.dy, bytes},  {p.dres, bytes},
+                                                {p.gamma, param}, {p.beta, param}, {p.mean, stat},
+                                                {p.rstd, stat}};
+  const std::pair<const void*, int64_t> out[] = {
+      {p.dx, bytes}, {dgamma, 4 * p.cols}, {dbeta, 4 * p.cols}};
+  for (const auto& o : out)
+    for (const auto& i : in)
+      if (overlaps(o.first, o.second, i.first, i.second)) return false;
+  return true;
+}
+
+int launch_backward_small(const BwdParams& p, int dtype, hipStream_t s) {
+  SmallArgs a{};
+  a.p = p;
+  const SmallPlan pl = plan(p, element_size(dtype));
+  if (pl.vpl == 0) return FLN_ERR_INVALID;
+  a.p.wpr = pl.wpr;
+  a.dx_blocks = pl.dx_blocks;
+  a.groups = pl.groups;
+  const int blocks = pl.dx_blocks + pl.col_blocks;
+  if (blocks == 0) return FLN_OK;
+  auto go = [&](auto t) {
+    using T = decltype(t);
+    switch (pl.vpl) {
+      case 1: return launch_vpl<T, 1>(a, blocks, s);
+      case 2: return launch_vpl<T, 2>(a, blocks, s);
+      case 4: return launch_vpl<T, 4>(a, blocks, s);
+      default: return launch_vpl<T, 8>(a, blocks, s);
+    }
+  };
+  switch (dtype) {
+    case FLN_F32: return go(float{});
+    case FLN_BF16: return go(__bf16{});
+    case FLN_F16: return go(_Float16{});
+    default: return FLN_ERR_INVALID;
+  }
+}
+
+}  // namespace fln

@@ -156,6 +156,31 @@ template <class T, int VEC> struct RaggedRow {
   }
 };
 
+// Stores elements e >= lo of a pack at byte offset off (lo = 0: all, 16 or 8 bytes at once).  For a
+// ragged row's last vector in kernels that read a row again while writing it: with the output in
+// place of the input, another thread may have overwritten the elements it shares with the vector
+// before it by the time this thread reads them.
+template <class T, int VEC, int POL>
+__device__ __forceinline__ void buf_store_own(const Pack<T, VEC>& p, rsrc_t r, uint32_t off,
+                                              int lo) {
+  if (lo == 0) {
+    buf_store_at<Pack<T, VEC>, POL>(p, r, off);
+  } else if (lo < VEC) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+      if (e >= lo) {
+        using IO = BufIO<sizeof(T), POL>;
+        IO::store(__builtin_bit_cast(typename IO::W, p.v[e]), r,
+                  off + e * static_cast<uint32_t>(sizeof(T)));
+      }
+  }
+}
+// Byte ranges [a, a + na) and [b, b + nb) overlap (null pointers never do).
+inline bool overlaps(const void* a, int64_t na, const void* b, int64_t nb) {
+  if (a == nullptr || b == nullptr) return false;
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x < y + static_cast<uintptr_t>(nb) && y < x + static_cast<uintptr_t>(na);
+}
 __device__ __forceinline__ void buf_store_f32(float x, rsrc_t r, uint32_t byte_off) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), r, byte_off, 0, 0);
 }

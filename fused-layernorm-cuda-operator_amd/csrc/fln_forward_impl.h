@@ -834,8 +834,13 @@ __global__ __launch_bounds__(kFwdLdsThreads) void fwd_lds_kernel(const FwdParams
 constexpr int kFwdWideThreads = 1024;
 constexpr int kFwdWideStepBytes = 64;  // bytes of the row per thread and step (4 vectors)
 
-template <class T, int FP8, bool RES, int GELU, int VEC, bool RAGGED>
-__global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdParams p) {
+// OWN (ragged rows with an output over an input): the row's last vector is written by element.
+template <class T, int FP8, bool RES, int GELU, int VEC, bool RAGGED, bool OWN = false>
+__global__ __launch_bounds__(kFwdWideThreads)
+// Ragged 16-bit LayerNorm / RMSNorm took 66 VGPRs, one block per CU: 2048 x 24001 80.4 us against 69.9
+// with two.
+__attribute__((amdgpu_waves_per_eu(RAGGED && !RES && !OWN && GELU == 0 && FP8 == 0 ? 8 : 4)))
+void fwd_wide_kernel(const FwdParams p) {
   constexpr int kT = kFwdWideThreads;
   constexpr int kW = kT / kWave;
   constexpr int U = kFwdWideStepBytes / (VEC * static_cast<int>(sizeof(T)));
@@ -908,8 +913,13 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
       const bool tail = RAGGED && base + kT * U > rag.nfull;  // uniform
       if constexpr (RES) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-          buf_store_at<P, FLN_FWD_STORE_POL>(hv[u], hr, off(base + t + kT * u));
+        for (int u = 0; u < U; ++u) {
+          const uint32_t v = base + t + kT * u;
+          if (OWN && tail)
+            buf_store_own<T, VEC, FLN_FWD_STORE_POL>(hv[u], hr, off(v), rag.lo(v));
+          else
+            buf_store_at<P, FLN_FWD_STORE_POL>(hv[u], hr, off(v));
+        }
       }
       if (p.rms) {
 #pragma unroll
@@ -1029,8 +1039,11 @@ __global__ __launch_bounds__(kFwdWideThreads) void fwd_wide_kernel(const FwdPara
           P o;
 #pragma unroll
           for (int e = 0; e < VEC; ++e) o.v[e] = from_f32<T>(a[e]);
-          buf_store_at<P, FLN_FWD_STORE_POL>(
-              o, make_rsrc(static_cast<T*>(p.y) + row * N, row_bytes), off(v));
+          const rsrc_t yr = make_rsrc(static_cast<T*>(p.y) + row * N, row_bytes);
+          if (OWN && base + kT * U > rag.nfull)  // uniform
+            buf_store_own<T, VEC, FLN_FWD_STORE_POL>(o, yr, off(v), rag.lo(v));
+          else
+            buf_store_at<P, FLN_FWD_STORE_POL>(o, yr, off(v));
         } else {
           float m = inv;
           if constexpr (FP8 == 2) {
@@ -1785,13 +1798,6 @@ int launch_split(FwdParams p, hipStream_t s) {
              fwd_split_out_kernel<T, FP8, false, 0, VEC, true>);
 }
 
-// Byte ranges [a, a + na) and [b, b + nb) overlap (null pointers never do).
-inline bool overlaps(const void* a, int64_t na, const void* b, int64_t nb) {
-  if (a == nullptr || b == nullptr) return false;
-  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-  return x < y + static_cast<uintptr_t>(nb) && y < x + static_cast<uintptr_t>(na);
-}
-
 template <class T, int FP8, int VEC, bool RAGGED>
 int launch_wide(const FwdParams& p, hipStream_t s) {
   auto launch = [&](auto kernel) {
@@ -1804,6 +1810,16 @@ int launch_wide(const FwdParams& p, hipStream_t s) {
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kFwdWideThreads), 0, s, p);
     return static_cast<int>(hipGetLastError());
   };
+  if constexpr (RAGGED && FP8 == 0) {
+    const int64_t bytes = p.rows * p.cols * static_cast<int64_t>(sizeof(T));
+    if (overlaps(p.y, bytes, p.x, bytes) || overlaps(p.y, bytes, p.res, bytes) ||
+        overlaps(p.h, bytes, p.x, bytes) || overlaps(p.h, bytes, p.res, bytes)) {
+      if (p.res) return launch(fwd_wide_kernel<T, 0, true, 0, VEC, true, true>);
+      if (p.gelu == FLN_GELU_ERF) return launch(fwd_wide_kernel<T, 0, false, 1, VEC, true, true>);
+      if (p.gelu == FLN_GELU_TANH) return launch(fwd_wide_kernel<T, 0, false, 2, VEC, true, true>);
+      return launch(fwd_wide_kernel<T, 0, false, 0, VEC, true, true>);
+    }
+  }
   if (p.res) return launch(fwd_wide_kernel<T, FP8, true, 0, VEC, RAGGED>);
   if constexpr (FP8 == 0) {
     if (p.gelu == FLN_GELU_ERF) return launch(fwd_wide_kernel<T, 0, false, 1, VEC, RAGGED>);

@@ -73,3 +73,34 @@ def test_ragged_outputs_stay_inside(lib, dtype, rows, cols):
             capi.check(call(out))
             assert (buf[:lead] == 7).all() and (buf[lead + n:] == 7).all()
             assert torch.equal(out.view(rows, cols), want)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("rows,cols", [(3, 600), (300, 1023), (7, 8193), (5, 20001), (300, 33001)])
+def test_ragged_in_place(lib, dtype, rows, cols):
+    """y over x and dx over dy: the outputs of separate buffers, bit for bit, also where the row's
+    last vector shares elements with the one before it."""
+    gen = torch.Generator().manual_seed(cols + 1)
+    x, dy = (cuda(torch.randn(rows, cols, generator=gen).to(dtype)) for _ in range(2))
+    g, b = (cuda(torch.randn(cols, generator=gen).to(dtype)) for _ in range(2))
+    p = capi.ptr
+    code, st = capi.dtype_code(x), capi.stream()
+    y0, mean, rstd = ln_forward(lib, x, g, b, 1e-5)
+    y = x.clone()
+    capi.check(lib.fln_layernorm_forward(p(y), p(g), p(b), p(y), None, None, rows, cols, code,
+                                         1e-5, st))
+    assert torch.equal(y, y0)
+    ws, nb = workspace(lib, rows, cols, x)
+    outs = []
+    for inplace in (False, True):
+        d = dy.clone()
+        dx = d if inplace else torch.empty_like(d)
+        dg, db = torch.empty(cols, device="cuda"), torch.empty(cols, device="cuda")
+        capi.check(lib.fln_layernorm_backward(p(d), p(x), p(mean), p(rstd), p(g), None, p(dx),
+                                              p(dg), p(db), rows, cols, code, capi.F32, p(ws), nb,
+                                              st))
+        outs.append((dx, dg, db))
+    ulp = {torch.float32: 2.0 ** -20, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+    for a, c in zip(*outs):  # another route may sum in another order: one rounding of the type
+        scale = c.float().abs().max()
+        assert (a.float() - c.float()).abs().max() <= (ulp if a.dtype == dtype else 1e-5) * scale
