@@ -58,15 +58,6 @@ __device__ __forceinline__ void add4(float4& a, const float4& b) {
   a.w += b.w;
 }
 
-__device__ __forceinline__ void store_param(void* out, int dtype, int64_t i, float v) {
-  if (dtype == FLN_F32)
-    static_cast<float*>(out)[i] = v;
-  else if (dtype == FLN_BF16)
-    static_cast<__bf16*>(out)[i] = from_f32<__bf16>(v);
-  else
-    static_cast<_Float16*>(out)[i] = from_f32<_Float16>(v);
-}
-
 __host__ __device__ inline int64_t quad_blocks(const ColReduceArgs& a) {
   const int64_t ld = (a.N + 3) & ~int64_t(3);
   return a.ny * (((ld >> 2) + kCrQuads - 1) / kCrQuads);
@@ -1560,6 +1551,16 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
         tun.bwd_colpass_per_cu > 0 ? tun.bwd_colpass_per_cu : FLN_COLPASS_BLOCKS_PER_CU;
     int64_t chunks = (per_cu * static_cast<int64_t>(device_cu_count()) + tiles - 1) / tiles;
     if (chunks > workspace_partial_rows(rows)) chunks = workspace_partial_rows(rows);
+    // Few rows: block rows of one batch of rows in flight, at most as many as the flat column
+    // reduction takes (a partial row per row cost its 32-slice form, and left the workspace no room
+    // for splits of the row statistics).  Backward calls, us: fp32 4 x
+    // 50000 21.5 -> 8.8, 26 x 38032 17.2 -> 13.2, 100 x 60000 36.8 -> 30.4; bf16 20 x 100000 26.4
+    // -> 16.2, 100 x 80000 33.6 -> 29.0; 128 x 131072 and 64 x 1048576 (8 and 1 already) equal.
+    if (rows <= 2 * kWideUnroll * kCrFlatMaxG) {
+      int64_t few = (rows + kWideUnroll - 1) / kWideUnroll;
+      if (few > kCrFlatMaxG) few = kCrFlatMaxG;
+      if (chunks > few) chunks = few;
+    }
     if (chunks < 1) chunks = 1;
     g.two_pass = true;
     g.threads = kWideThreads;
@@ -1597,7 +1598,11 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
   // gradient is requested, then the row statistics of the two-pass path [rows, splits, 2]
   // (16-byte aligned: ld is a multiple of 4).  At most fln_backward_workspace_bytes() (blocks <=
   // workspace_partial_rows on every path; splits within what that bound leaves).
-  const int64_t part = (dgamma || dbeta) ? 2 * geo.blocks * ld : 0;
+  // A column pass with one block row (columns >= 2 x CUs column tiles, or at most 8 rows) holds the
+  // final column sums: it writes dgamma / dbeta itself, without partial rows or the column
+  // reduction (the same bits: the reduction of one partial row only converts it).
+  const bool direct = geo.two_pass && geo.blocks == 1;
+  const int64_t part = (dgamma || dbeta) && !direct ? 2 * geo.blocks * ld : 0;
   // Row statistics of the two-pass path: fewer rows than the statistics pass has blocks split
   // into column chunks of whole steps (kWideUnroll x kWideThreads vectors), as many as the
   // workspace bound (fln_backward_workspace_bytes, not the size passed, so that the split and
@@ -1607,10 +1612,14 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
   const int64_t nvec = (p.cols + geo.vec - 1) / geo.vec;
   p.stat_chunk = nvec;
   if (geo.two_pass) {
-    constexpr int64_t step = int64_t(kWideUnroll) * kWideThreads;
-    const int64_t steps = (nvec + step - 1) / step;
     const int forced = tuning().bwd_stat_splits;  // FLN_BWD_STAT_SPLITS
     const int64_t items = kRowstatItemsPerCu * static_cast<int64_t>(device_cu_count());
+    // Whole steps of the statistics pass, or a quarter of one where rows x steps are too few for
+    // every CU (with the rule on block rows below, backward calls, us: bf16 2 x
+    // 100001 47.7 -> 12.0, fp32 4 x 50000 21.5 -> 8.8).
+    int64_t step = int64_t(kWideUnroll) * kWideThreads;
+    if (p.rows * ((nvec + step - 1) / step) < items) step /= 4;
+    const int64_t steps = (nvec + step - 1) / step;
     splits = forced > 0 ? forced : (items + p.rows - 1) / p.rows;
     if (splits > kMaxStatSplits) splits = kMaxStatSplits;
     const int64_t bound = 2 * workspace_partial_rows(p.rows) * ld + 2 * p.rows;
@@ -1628,13 +1637,22 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
                         sizeof(float);
     if (need > workspace_bytes) return FLN_ERR_TOO_LARGE;
   }
+  if ((dgamma || dbeta) && dparam_dtype != FLN_F32 && dparam_dtype != FLN_BF16 &&
+      dparam_dtype != FLN_F16)
+    return FLN_ERR_INVALID;
+  if (backward_is_small(p, dgamma, dbeta, dtype)) {
+    p.out_g = dgamma;
+    p.out_b = dbeta;
+    p.out_dtype = dparam_dtype;
+    p.part_g = p.part_b = nullptr;
+    if (tuning().debug_geometry)
+      fprintf(stderr, "fln backward: rows=%lld cols=%lld -> small\n",
+              static_cast<long long>(p.rows), static_cast<long long>(p.cols));
+    return launch_backward_small(p, dtype, s);
+  }
   p.part_g = dgamma ? ws : nullptr;
   p.part_b = dbeta ? ws + geo.blocks * ld : nullptr;
   p.rowstat = have_workspace ? ws + part : nullptr;
-  // The column pass with a single block row (columns >= 2 x CUs column tiles) holds the final
-  // column sums: it writes dgamma / dbeta itself and the column reduction is skipped (the same
-  // bits: the reduction of one partial row only converts it; 64 x 1048576 bf16: 6.4 us).
-  const bool direct = geo.two_pass && geo.blocks == 1;
   if (direct) {
     p.out_g = dgamma;
     p.out_b = dbeta;
@@ -1647,9 +1665,6 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
   a.G = geo.blocks;
   a.N = p.cols;
   a.out_dtype = dparam_dtype;
-  if (a.ny > 0 && dparam_dtype != FLN_F32 && dparam_dtype != FLN_BF16 &&
-      dparam_dtype != FLN_F16)
-    return FLN_ERR_INVALID;
   int rc;
   switch (dtype) {
     case FLN_F32: rc = dispatch_backward<float>(p, geo, s); break;

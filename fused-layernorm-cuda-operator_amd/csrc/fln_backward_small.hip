@@ -8,9 +8,18 @@
 //   dx blocks (the first p.dx_blocks): whole rows, each in the registers of `wpr` waves, up to 8
 //     vectors per lane in the I/O type (65536 16-bit or 32768 fp32 columns: without column sums to
 //     carry, a 1024-thread block holds x and dy of a row that wide); as bwd_reg_kernel otherwise.
-//   column blocks: 64 vector columns each, one per lane, over every row: 16 waves take every 16th
-//     row with 8 in flight, then the 16 partial sums of a column are added in order through LDS.
+//   column blocks: `cw` vector columns each (8 to 64, one per lane) over every row: the block's
+//     1024 / cw row slices take the rows in turn, 4 in flight each, then the slices' partial sums
+//     of a column are added in order through LDS.
 // Both roles take unaligned vectors (RaggedRow), so any width of at least one vector runs here.
+//
+// Taken for at most one row per CU.  Backward calls, us, before -> here: fp32 32 x 768 6.4 -> 3.6, 128
+// x 768 6.9 -> 4.1, 256 x 768 7.7 -> 4.7, 256 x 16384 27.4 -> 18.2, 256 x 32768 36.8 -> 36.5; bf16 64 x
+// 4096 8.1 -> 4.3, 256 x 1024 8.4 -> 4.8, 256 x 8192 19.5 -> 8.1, 200 x 12288 19.9 -> 7.6, 100 x 40000
+// 25.3 -> 14.7, 1 x 65536 15.3 -> 11.8; erf GELU 64 x 4096 9.5 -> 8.2, 100 x 30000 32.3 -> 15.3, 256 x
+// 20000 34.2 / 34.4; residual gradient 200 x 50000 41.1 -> 28.2.  More rows amortize the two stages'
+// overhead and read x and dy once.  What bounds it: one launch and two dependent round trips to memory
+// for narrow rows; the bandwidth of the few CUs that hold a row for wide ones.
 #include <type_traits>
 
 #include "fln_device.h"
@@ -26,6 +35,7 @@ struct SmallArgs {
   BwdParams p;
   int dx_blocks;  // blocks of the dx role (0: dx not requested)
   int groups;     // row groups per dx block
+  int cw;         // vector columns of a column block
 };
 
 template <class T, bool DRES, int GELU, int VEC, int VPL>
@@ -166,12 +176,19 @@ __global__ __launch_bounds__(kSmallThreads) void bwd_small_kernel(const SmallArg
     return;
   }
 
-  // Column role.  Rows in flight per wave: 8 (4 with GELU on 8 columns, which spilled).
-  constexpr int kColUnroll = GELU != 0 && VEC == 8 ? 4 : 8;
-  constexpr int kCols = kWave * VEC;  // columns of a block
-  __shared__ float part[2][kSmallWaves][kCols];
-  const uint32_t v0 = (blockIdx.x - static_cast<uint32_t>(a.dx_blocks)) * kWave;
-  const uint32_t off = rag.off(v0 + lane);
+  // Column role: lane = (row slice of the wave, vector column).
+  constexpr int kRows = 4;               // rows in flight per lane
+  constexpr int kMostCols = kWave * VEC; // columns of a block at most
+  __shared__ float part[2][kSmallWaves * kMostCols];
+  const int cw = a.cw;
+  const int col = lane & (cw - 1), slices = kSmallWaves * (kWave / cw);
+  const int slice = wave * (kWave / cw) + lane / cw;
+  const uint32_t v0 = (blockIdx.x - static_cast<uint32_t>(a.dx_blocks)) * cw;
+  const uint32_t off = rag.off(v0 + col);
+  // One resource over each tensor (under 2 GiB here): the lanes of a wave take different rows.
+  const uint32_t rows = static_cast<uint32_t>(p.rows);
+  const rsrc_t xr = make_rsrc(X, rows * row_bytes), dr = make_rsrc(DY, rows * row_bytes);
+  const rsrc_t mr = make_rsrc(p.rms ? nullptr : p.mean, rows * 4u), sr = make_rsrc(p.rstd, rows * 4u);
   const P gv = buf_load_at<P>(g_rs, off);
   P bv{};
   if constexpr (GELU != 0) {
@@ -181,23 +198,23 @@ __global__ __launch_bounds__(kSmallThreads) void bwd_small_kernel(const SmallArg
   float acc_g[VEC], acc_b[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) acc_g[e] = acc_b[e] = 0.0f;
-  for (int64_t row = wave; row < p.rows; row += kColUnroll * kSmallWaves) {
-    P xv[kColUnroll], dv[kColUnroll];
-    float mu[kColUnroll], rs[kColUnroll];
+  for (uint32_t row0 = 0; row0 < rows; row0 += kRows * slices) {
+    P xv[kRows], dv[kRows];
+    float mu[kRows], rs[kRows];
 #pragma unroll
-    for (int u = 0; u < kColUnroll; ++u) {
+    for (int u = 0; u < kRows; ++u) {
       // Rows past the tensor read as zeros, statistics included: they add exact zeros.
-      const bool in = row + u * kSmallWaves < p.rows;  // uniform
-      const int64_t r = in ? row + u * kSmallWaves : row;
-      const uint32_t nb = in ? row_bytes : 0u, sb = in ? 4u : 0u;
-      xv[u] = buf_load_at<P>(make_rsrc(X + r * N, nb), off);
-      dv[u] = buf_load_at<P>(make_rsrc(DY + r * N, nb), off);
-      mu[u] = __builtin_bit_cast(
-          float, BufIO<4>::load(make_rsrc(p.rms ? nullptr : p.mean + r, sb), 0));
-      rs[u] = __builtin_bit_cast(float, BufIO<4>::load(make_rsrc(p.rstd + r, sb), 0));
+      const uint32_t r = row0 + u * slices + slice;
+      const bool in = r < rows;
+      const uint32_t o = in && off != kOutOfRange ? r * row_bytes + off : kOutOfRange;
+      const uint32_t so = in ? r * 4u : kOutOfRange;
+      xv[u] = buf_load_at<P>(xr, o);
+      dv[u] = buf_load_at<P>(dr, o);
+      mu[u] = __builtin_bit_cast(float, BufIO<4>::load(mr, so));
+      rs[u] = __builtin_bit_cast(float, BufIO<4>::load(sr, so));
     }
 #pragma unroll
-    for (int u = 0; u < kColUnroll; ++u)
+    for (int u = 0; u < kRows; ++u)
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         const float xh = (to_f32(xv[u].v[e]) - mu[u]) * rs[u];
@@ -207,20 +224,20 @@ __global__ __launch_bounds__(kSmallThreads) void bwd_small_kernel(const SmallArg
         acc_b[e] += d;
       }
   }
+  const int cols = cw * VEC;  // columns of this block
 #pragma unroll
   for (int e = 0; e < VEC; ++e) {
-    part[0][wave][lane * VEC + e] = acc_g[e];
-    part[1][wave][lane * VEC + e] = acc_b[e];
+    part[0][slice * cols + col * VEC + e] = acc_g[e];
+    part[1][slice * cols + col * VEC + e] = acc_b[e];
   }
   __syncthreads();
-  if (threadIdx.x >= 2 * kCols) return;
-  const int which = threadIdx.x / kCols, c = threadIdx.x % kCols;
+  if (static_cast<int>(threadIdx.x) >= 2 * cols) return;
+  const int which = static_cast<int>(threadIdx.x) / cols, c = static_cast<int>(threadIdx.x) % cols;
   const uint32_t v = v0 + static_cast<uint32_t>(c / VEC);
   void* out = which == 0 ? p.out_g : p.out_b;
   if (out == nullptr || c % VEC < rag.lo(v)) return;  // (lo = VEC past the row)
-  float s = part[which][0][c];
-#pragma unroll
-  for (int k = 1; k < kSmallWaves; ++k) s += part[which][k][c];
+  float s = part[which][c];
+  for (int k = 1; k < slices; ++k) s += part[which][k * cols + c];
   store_param(out, p.out_dtype, rag.off(v) / static_cast<uint32_t>(sizeof(T)) + c % VEC, s);
 }
 
@@ -248,7 +265,7 @@ int launch_vpl(const SmallArgs& a, int blocks, hipStream_t s) {
 }
 
 struct SmallPlan {
-  int wpr, vpl, groups, dx_blocks, col_blocks;
+  int wpr, vpl, groups, dx_blocks, col_blocks, cw;
 };
 
 // Waves per row (1..16) and vectors per lane (1, 2, 4 or 8) of the dx role; vpl 0: too wide.
@@ -260,7 +277,11 @@ SmallPlan plan(const BwdParams& p, int es) {
   s.vpl = slots <= 16 ? 1 : slots <= 32 ? 2 : slots <= 64 ? 4 : slots <= 128 ? 8 : 0;
   if (s.vpl == 0) return s;
   s.wpr = static_cast<int>((slots + s.vpl - 1) / s.vpl);
-  s.col_blocks = p.out_g || p.out_b ? static_cast<int>(slots) : 0;
+  // Column blocks: fewer columns and more row slices each while a slice has more than 4 rows, the
+  // blocks leaving most CUs to the rows.
+  s.cw = kWave;
+  while (s.cw > 8 && p.rows * s.cw > 4 * kSmallThreads && nvec <= 64 * (s.cw / 2)) s.cw /= 2;
+  if (p.out_g || p.out_b) s.col_blocks = static_cast<int>((nvec + s.cw - 1) / s.cw);
   if (p.dx) {
     // One row per block while the blocks still fit the CUs, then as many as a block holds.
     const int64_t room = cus > 2 * s.col_blocks ? cus - s.col_blocks : cus / 2;
@@ -271,13 +292,6 @@ SmallPlan plan(const BwdParams& p, int es) {
     s.dx_blocks = static_cast<int>((p.rows + groups - 1) / groups);
   }
   return s;
-}
-
-// Byte ranges [a, a + na) and [b, b + nb) overlap (null pointers never do).
-bool overlaps(const void* a, int64_t na, const void* b, int64_t nb) {
-  if (a == nullptr || b == nullptr) return false;
-  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-  return x < y + static_cast<uintptr_t>(nb) && y < x + static_cast<uintptr_t>(na);
 }
 
 }  // namespace
@@ -292,7 +306,7 @@ bool backward_is_small(const BwdParams& p, const void* dgamma, const void* dbeta
   const int64_t vec = 16 / es;
   if (p.cols < vec || p.cols > 16 * kWave * 8 * vec) return false;
   const int64_t limit = tun.bwd_small_rows > 0 ? tun.bwd_small_rows : device_cu_count();
-  if (p.rows > limit) return false;
+  if (p.rows > limit || p.rows * p.cols * es >= int64_t(1) << 31) return false;
   // The roles run at the same time: an output in place of an input (dx over dy, say) would be
   // written while other blocks still read it.
   const int64_t bytes = p.rows * p.cols * es, param = p.cols * es, stat = p.rows * 4;
@@ -315,6 +329,7 @@ int launch_backward_small(const BwdParams& p, int dtype, hipStream_t s) {
   a.p.wpr = pl.wpr;
   a.dx_blocks = pl.dx_blocks;
   a.groups = pl.groups;
+  a.cw = pl.cw;
   const int blocks = pl.dx_blocks + pl.col_blocks;
   if (blocks == 0) return FLN_OK;
   auto go = [&](auto t) {

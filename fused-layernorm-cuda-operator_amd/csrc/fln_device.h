@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "../../include/fused_layernorm.h"
 #include "fln_gelu_table.h"
 
 namespace fln {
@@ -183,6 +184,16 @@ inline bool overlaps(const void* a, int64_t na, const void* b, int64_t nb) {
 }
 __device__ __forceinline__ void buf_store_f32(float x, rsrc_t r, uint32_t byte_off) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), r, byte_off, 0, 0);
+}
+
+// Element i of a parameter gradient, rounded once to its type (an FLN_* code).
+__device__ __forceinline__ void store_param(void* out, int dtype, int64_t i, float v) {
+  if (dtype == FLN_F32)
+    static_cast<float*>(out)[i] = v;
+  else if (dtype == FLN_BF16)
+    static_cast<__bf16*>(out)[i] = from_f32<__bf16>(v);
+  else
+    static_cast<_Float16*>(out)[i] = from_f32<_Float16>(v);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -78,7 +78,7 @@ int device_cu_count() {
 // Tuning and debugging knobs: getenv scans the whole environment (~0.1 us each with ~100
 // variables), so the knobs are read once, at the first launch, into a snapshot that
 // fln_reload_tuning() replaces.  Replaced snapshots are never freed (a concurrent launch may
-// still be reading one; each is 44 bytes and only tests and tuning sweeps reload).
+// still be reading one; each is under 100 bytes and only tests and tuning sweeps reload).
 namespace {
 int env_knob(const char* name, int dflt) {
   const char* v = getenv(name);
@@ -105,6 +105,7 @@ Tuning read_tuning() {
   t.bwd_no_two_pass = env_knob("FLN_BWD_NO_TWO_PASS", 0);
   t.bwd_stat_splits = env_knob("FLN_BWD_STAT_SPLITS", 0);
   t.bwd_colpass_per_cu = env_knob("FLN_BWD_COLPASS_PER_CU", 0);
+  t.bwd_small_rows = env_knob("FLN_BWD_SMALL_ROWS", 0);
   return t;
 }
 

@@ -139,6 +139,7 @@ struct Tuning {
   int bwd_no_two_pass; // FLN_BWD_NO_TWO_PASS: never the two-pass backward
   int bwd_stat_splits; // FLN_BWD_STAT_SPLITS: column splits per row of the two-pass statistics
   int bwd_colpass_per_cu; // FLN_BWD_COLPASS_PER_CU: column-pass blocks per CU (two-pass path)
+  int bwd_small_rows;  // FLN_BWD_SMALL_ROWS: row limit of the one-launch backward (negative: never)
 };
 const Tuning& tuning();  // read at the first call; fln_reload_tuning() reads again
 void reload_tuning();
@@ -148,6 +149,12 @@ int launch_forward(const FwdParams& p, int dtype, bool out_fp8, hipStream_t s);
 // geometry needs more returns FLN_ERR_TOO_LARGE before anything is launched.
 int launch_backward(const BwdParams& p, int dtype, void* dgamma, void* dbeta, int dparam_dtype,
                     bool have_workspace, size_t workspace_bytes, hipStream_t s);
+
+// The backward of few rows in one launch without a workspace (fln_backward_small.hip): whether a
+// call takes it (any alignment; no output over an input; never while another backward knob is
+// set), and the launch.
+bool backward_is_small(const BwdParams& p, const void* dgamma, const void* dbeta, int dtype);
+int launch_backward_small(const BwdParams& p, int dtype, hipStream_t s);
 
 // Stage-1 geometry of the backward (shared by workspace sizing and the launch).
 struct BwdGeometry {

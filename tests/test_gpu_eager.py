@@ -72,9 +72,17 @@ def test_eager_paths_equal_the_operators(monkeypatch, kind, dtype, lead, shape, 
             m.setattr(fops, "_ordinary", lambda *t: False)
             want = _step(kind, x, r, shape, w, b, use)
         for a, c in zip(got[0] + list(got[1]), want[0] + list(want[1])):
-            # The operator path materializes the gradient of an unused output as zeros.
             assert (a is None) == (c is None)
-            assert a is None or (a.shape == c.shape and torch.equal(a, c)), kind
+            if a is None or (a.shape == c.shape and torch.equal(a, c)):
+                continue
+            # The operators fill in zeros for the gradient of an unused h and add them in the
+            # kernel's residual form, which rounds the sum to fp32 before the output type; without
+            # them the last FMA rounds to the output type directly.  Both are within half an ulp
+            # plus half an fp32 ulp of the same value, so at most one ulp apart.
+            assert use == (True, False) and a.shape == c.shape, kind
+            ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+            err = (a.float() - c.float()).abs()
+            assert (err <= ulp * c.float().abs() + 2.0 ** -24).all() and dtype != torch.float32
 
 
 @pytest.mark.parametrize("kind", ["gelu_tanh", "add_rms"])
