@@ -727,7 +727,14 @@ __global__ __launch_bounds__(NT) void bwd_lds_kernel(const BwdParams p) {
 //     accumulates dgamma / dbeta in registers, then writes one partial row per block row for
 //     col_reduce_kernel.
 // 5 streams (x, dy twice, dx once) instead of 3, but every access is a coalesced vector stream
-// and no thread holds more than eight vectors per array.
+// and no thread holds more than eight vectors per array.  The row statistics read x and dy with
+// the default cache policy, so that the column pass, which reads them for the last time and
+// streams, finds in the 256 MB memory-side cache what fits there (backward calls, us, streaming
+// loads in the first pass / default there / default in both: fp32 256 x 65536 60.8 / 58.4 / 61.9,
+// 1000 x 20001 87.4 / 79.8 / 80.4; bf16 300 x 100000 84.3 / 78.5 / 78.4, 2048 x 40000 164.5 /
+// 155.2 / 168.4, 8192 x 40000 632 / 618 / -, 64 x 1048576 114.0 / 115.3 / 119.0).  The column
+// pass taking the rows from the last one on, so as to start on those read last, measured no
+// better than in order (155.2 -> 154.8, 618 -> 626, fp32 4096 x 20480 296 -> 303).
 constexpr int kWideThreads = 256;
 // Rows (column pass) or vector steps (row statistics) in flight per thread: 8 rather than 4
 // measured 2-4% faster with few rows (bf16 backward calls, us: 128 x 131072 43.1 -> 41.2, 512 x
@@ -788,8 +795,8 @@ __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdPara
         const uint32_t o = !RAGGED   ? static_cast<uint32_t>(v) * static_cast<uint32_t>(sizeof(P))
                            : v < v_hi ? rag.off(static_cast<uint32_t>(v))
                                       : kOutOfRange;
-        xv[u] = buf_load_at<P, kStream>(xr, o);
-        dv[u] = buf_load_at<P, kStream>(dr, o);
+        xv[u] = buf_load_at<P>(xr, o);
+        dv[u] = buf_load_at<P>(dr, o);
         gv[u] = buf_load_at<P>(gr, o);
         if constexpr (GELU != 0) bv[u] = buf_load_at<P>(br, o);
       }
