@@ -802,6 +802,8 @@ __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdPara
       }
 #pragma unroll
       for (int u = 0; u < kWideUnroll; ++u) {
+        if constexpr (GELU != 0)  // no thread of the block has a vector left (uniform)
+          if (v0 - t + u * kWideThreads >= v_hi) break;
         // A ragged row's last vector counts only its own elements.
         if (RAGGED && v0 + u * kWideThreads == nvec - 1) {
 #pragma unroll
@@ -835,7 +837,8 @@ __global__ __launch_bounds__(kWideThreads) void bwd_rowstat_kernel(const BwdPara
   }
 }
 
-// OWN (ragged rows with dx over an input): the row's last vector is written by element.
+// OWN (ragged rows with dx over an input): the row's last vector is written by element.  VEC: 16
+// bytes, or 4 for few rows (backward_geometry; ragged and OWN, which hold for any width).
 template <class T, bool DRES, int GELU, int VEC, bool RAGGED, bool OWN = false>
 __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdParams p,
                                                                    const float2* stats) {
@@ -895,6 +898,10 @@ __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdPara
 #pragma unroll
     for (int u = 0; u < kWideUnroll; ++u) {
       const bool in = row + u * G < p.rows;
+      // Rows past the tensor, a uniform branch (whole vectors without GELU: it cost more than the
+      // work it skips, fp32 30 x 60001 14.4 -> 14.7 us).
+      if constexpr (GELU != 0 || VEC * sizeof(T) < 16)
+        if (!in) break;
       const int64_t r = in ? row + u * G : row;
       P o;
 #pragma unroll
@@ -934,7 +941,7 @@ __global__ __launch_bounds__(kWideThreads) void bwd_colpass_kernel(const BwdPara
   }
   const int64_t ld = (N + 3) & ~int64_t(3);
   const int64_t c = static_cast<int64_t>(blockIdx.y) * ld + col;
-  if constexpr (RAGGED) {
+  if constexpr (RAGGED && VEC % 4 == 0) {
     if (lo == 0) {
       if (p.part_g) store_columns<VEC>(p.part_g + c, acc_g);
       if (p.part_b) store_columns<VEC>(p.part_b + c, acc_b);
@@ -1206,6 +1213,28 @@ int launch_two_pass(const BwdParams& p, const BwdGeometry& geo, hipStream_t s) {
   const int64_t nvec = (p.cols + VEC - 1) / VEC;
   const dim3 g2(static_cast<unsigned>((nvec + kWideThreads - 1) / kWideThreads),
                 static_cast<unsigned>(geo.blocks));
+  if (geo.col_vec < VEC) {  // few rows: a quarter of a vector per thread in the column pass
+    constexpr int CV = VEC / 4;
+    const int64_t cvec = (p.cols + CV - 1) / CV;
+    const dim3 g4(static_cast<unsigned>((cvec + kWideThreads - 1) / kWideThreads),
+                  static_cast<unsigned>(geo.blocks));
+    auto run = [&](auto rowstat, auto colpass) {
+      hipLaunchKernelGGL(rowstat, g1, blk, 0, s, p, stats);
+      hipLaunchKernelGGL(colpass, g4, blk, 0, s, p, stats);
+      return static_cast<int>(hipGetLastError());
+    };
+    if (p.gelu == 1)
+      return run(bwd_rowstat_kernel<T, 1, VEC, RAGGED>,
+                 bwd_colpass_kernel<T, false, 1, CV, true, true>);
+    if (p.gelu == 2)
+      return run(bwd_rowstat_kernel<T, 2, VEC, RAGGED>,
+                 bwd_colpass_kernel<T, false, 2, CV, true, true>);
+    if (p.dres)
+      return run(bwd_rowstat_kernel<T, 0, VEC, RAGGED>,
+                 bwd_colpass_kernel<T, true, 0, CV, true, true>);
+    return run(bwd_rowstat_kernel<T, 0, VEC, RAGGED>,
+               bwd_colpass_kernel<T, false, 0, CV, true, true>);
+  }
   if constexpr (RAGGED) {
     const int64_t bytes = p.rows * p.cols * static_cast<int64_t>(sizeof(T));
     if (overlaps(p.dx, bytes, p.x, bytes) || overlaps(p.dx, bytes, p.dy, bytes) ||
@@ -1569,6 +1598,22 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
       if (chunks > few) chunks = few;
     }
     if (chunks < 1) chunks = 1;
+    // Still fewer blocks than CUs and at most two (16-bit: four) batches of rows: a quarter of a
+    // vector per thread, so four times the blocks for the same work (any alignment: 4-byte
+    // accesses), and no more block rows than give 2 blocks per CU.  A chain of a few rows' loads,
+    // GELU derivatives and stores bounds such a call, not bandwidth.  Backward calls, us, whole
+    // vectors -> quarters: bf16 4 x 50000 LN 10.6 -> 8.4, residual gradient 11.3 -> 8.5, 16 x
+    // 200000 LN 16.2 -> 14.0; fp32 8 x 20001 9.6 -> 8.5, 16 x 60001 13.1 -> 12.0; erf GELU (with
+    // the row statistics' early exit) bf16 4 x 60001 16.9 -> 10.0, 16 x 50000 18.8 -> 13.1.  More
+    // rows have the blocks (fp32 30 x 60001 residual 16.1 -> 17.7, bf16 64 x 60001 21.7 -> 23.3).
+    g.col_vec = g.vec;
+    const int64_t batch = es == 2 ? kWideUnroll : 2 * kWideUnroll;
+    if (rows <= (es == 2 ? 4 : 2) * kWideUnroll && tiles * chunks <= device_cu_count()) {
+      g.col_vec = g.vec / 4;
+      const int64_t fill = 2 * static_cast<int64_t>(device_cu_count()) / (4 * tiles);
+      chunks = (rows + batch - 1) / batch;
+      if (chunks > fill) chunks = fill < 1 ? 1 : fill;
+    }
     g.two_pass = true;
     g.threads = kWideThreads;
     g.rows_per_block = (rows + chunks - 1) / chunks;

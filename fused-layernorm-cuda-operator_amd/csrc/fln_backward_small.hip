@@ -10,14 +10,14 @@
 //     carry, a 1024-thread block holds x and dy of a row that wide); as bwd_reg_kernel otherwise.
 //   column blocks: `cw` vector columns each (8 to 64, one per lane) over every row: the block's
 //     1024 / cw row slices take the rows in turn, 4 in flight each, then the slices' partial sums
-//     of a column are added in order through LDS.
+//     of a column are added through LDS.
 // Both roles take unaligned vectors (RaggedRow), so any width of at least one vector runs here.
 //
 // Taken for at most one row per CU.  Backward calls, us, before -> here: fp32 32 x 768 6.4 -> 3.6, 128
 // x 768 6.9 -> 4.1, 256 x 768 7.7 -> 4.7, 256 x 16384 27.4 -> 18.2, 256 x 32768 36.8 -> 36.5; bf16 64 x
 // 4096 8.1 -> 4.3, 256 x 1024 8.4 -> 4.8, 256 x 8192 19.5 -> 8.1, 200 x 12288 19.9 -> 7.6, 100 x 40000
-// 25.3 -> 14.7, 1 x 65536 15.3 -> 11.8; erf GELU 64 x 4096 9.5 -> 8.2, 100 x 30000 32.3 -> 15.3, 256 x
-// 20000 34.2 / 34.4; residual gradient 200 x 50000 41.1 -> 28.2.  More rows amortize the two stages'
+// 25.3 -> 14.7, 1 x 32768 11.5 -> 6.7; erf GELU 64 x 4096 9.5 -> 8.0, 100 x 30000
+// 32.3 -> 15.2; residual gradient 200 x 50000 41.1 -> 28.2.  More rows amortize the two stages'
 // overhead and read x and dy once.  What bounds it: one launch and two dependent round trips to memory
 // for narrow rows; the bandwidth of the few CUs that hold a row for wide ones.
 #include <type_traits>
@@ -213,16 +213,21 @@ __global__ __launch_bounds__(kSmallThreads) void bwd_small_kernel(const SmallArg
       mu[u] = __builtin_bit_cast(float, BufIO<4>::load(mr, so));
       rs[u] = __builtin_bit_cast(float, BufIO<4>::load(sr, so));
     }
+    // The rows in flight are summed by themselves first: shorter chains, smaller rounding errors.
 #pragma unroll
-    for (int u = 0; u < kRows; ++u)
+    for (int e = 0; e < VEC; ++e) {
+      float sum_g = 0.0f, sum_b = 0.0f;
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) {
+      for (int u = 0; u < kRows; ++u) {
         const float xh = (to_f32(xv[u].v[e]) - mu[u]) * rs[u];
         const float d = upstream(to_f32(dv[u].v[e]), xh, has_g ? to_f32(gv.v[e]) : 1.0f,
                                  GELU ? to_f32(bv.v[e]) : 0.0f);
-        acc_g[e] = fmaf(d, xh, acc_g[e]);
-        acc_b[e] += d;
+        sum_g = fmaf(d, xh, sum_g);
+        sum_b += d;
       }
+      acc_g[e] += sum_g;
+      acc_b[e] += sum_b;
+    }
   }
   const int cols = cw * VEC;  // columns of this block
 #pragma unroll
@@ -236,9 +241,14 @@ __global__ __launch_bounds__(kSmallThreads) void bwd_small_kernel(const SmallArg
   const uint32_t v = v0 + static_cast<uint32_t>(c / VEC);
   void* out = which == 0 ? p.out_g : p.out_b;
   if (out == nullptr || c % VEC < rag.lo(v)) return;  // (lo = VEC past the row)
-  float s = part[which][c];
-  for (int k = 1; k < slices; ++k) s += part[which][k * cols + c];
-  store_param(out, p.out_dtype, rag.off(v) / static_cast<uint32_t>(sizeof(T)) + c % VEC, s);
+  // Eight sums and a tree over them (slices is a multiple of 16): shorter chains, closer to the
+  // exact sum than the slices in turn.
+  float s[8] = {};
+  for (int k = 0; k < slices; k += 8)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s[j] += part[which][(k + j) * cols + c];
+  const float sum = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+  store_param(out, p.out_dtype, rag.off(v) / static_cast<uint32_t>(sizeof(T)) + c % VEC, sum);
 }
 
 template <class T, int VPL>
@@ -307,6 +317,22 @@ bool backward_is_small(const BwdParams& p, const void* dgamma, const void* dbeta
   if (p.cols < vec || p.cols > 16 * kWave * 8 * vec) return false;
   const int64_t limit = tun.bwd_small_rows > 0 ? tun.bwd_small_rows : device_cu_count();
   if (p.rows > limit || p.rows * p.cols * es >= int64_t(1) << 31) return false;
+  // The widest rows (8 vectors per lane) are bound by the one CU that holds a row: with a few rows
+  // the two passes spread each over many CUs (backward calls, us, here / two passes: bf16 LN 4 x
+  // 50000 11.8 / 8.4, 16 x 50000 12.2 / 12.0, 30 x 50000 12.6 / 15.0, off the 16-byte grid 4 x 60001
+  // 15.4 / 9.4, 16 x 60001 15.8 / 13.2, 30 x 60001 16.2 / 15.6; fp32 4 x 32768 8.5 / 7.2, 16 x 20001
+  // 8.2 / 10.4, 16 x 32768 8.8 / 10.6).
+  // So are 16-bit rows with GELU, whose derivative is taken twice per element: 8 vectors per lane
+  // never (64 x 50000 24.5 / 21.2, 128 x 50000 28.3 / 28), 4 only while every block has its own CU
+  // (200 x 20000 23.1 / 31.6, but 256 x 20000 35.4 / 34.2, 256 x 32768 38.1 / 33.1).
+  const int64_t nvec = (p.cols + vec - 1) / vec;
+  if (nvec > 64 * kWave) {
+    if (p.gelu && es == 2) return false;
+    if (p.rows < (es == 2 && p.cols % vec != 0 ? 32 : 16)) return false;
+  } else if (nvec > 32 * kWave && p.gelu && es == 2 &&
+             p.rows + (nvec + kWave - 1) / kWave > device_cu_count()) {
+    return false;
+  }
   // The roles run at the same time: an output in place of an input (dx over dy, say) would be
   // written while other blocks still read it.
   const int64_t bytes = p.rows * p.cols * es, param = p.cols * es, stat = p.rows * 4;

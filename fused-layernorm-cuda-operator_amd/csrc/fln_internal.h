@@ -162,6 +162,7 @@ struct BwdGeometry {
   int lds_cpt;    // > 0: rows staged through LDS, this many vectors per thread (reg_path false)
   bool two_pass;  // row statistics pass + column pass (rows past the register / LDS tiles)
   int vec;        // elements per vector access
+  int col_vec;    // two-pass: elements per access of the column pass
   bool ragged;    // rows off the 16-byte grid: unaligned vectors
   int vpl;        // vectors per lane (power of two, <= 16)
   int wpr;        // waves per row

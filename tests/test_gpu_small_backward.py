@@ -41,6 +41,16 @@ def test_small_backward(lib, kind, dtype, rows, cols, shifted):
     checks.test_random_shapes_against_the_oracle(lib, kind, dtype, rows, cols, shifted)
 
 
+# Around the rows and widths at which the two passes take over from the one launch, and those of
+# their column pass over quarters of a vector (1 to 3 elements past its tiles and vectors).
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 15, 16, 17, 31, 33])
+@pytest.mark.parametrize("kind,dtype,cols", [
+    ("ln", torch.bfloat16, 33281), ("ln_dres", torch.float16, 40960), ("gelu_none", torch.bfloat16,
+     32770), ("gelu_tanh", torch.float32, 16643), ("rms", torch.float32, 20481)])
+def test_few_wide_rows(lib, kind, dtype, rows, cols):
+    checks.test_random_shapes_against_the_oracle(lib, kind, dtype, rows, cols, rows % 2 == 1)
+
+
 def _backward(lib, dy, x, mean, rstd, g, want, ws=True, dx=None):
     rows, cols = x.shape
     p = capi.ptr
@@ -54,7 +64,7 @@ def _backward(lib, dy, x, mean, rstd, g, want, ws=True, dx=None):
     return dx, dg, db
 
 
-@pytest.mark.parametrize("rows,cols", [(17, 1023), (256, 768), (3, 40000), (300, 768)])
+@pytest.mark.parametrize("rows,cols", [(17, 1023), (256, 768), (20, 40000), (300, 768)])
 def test_small_backward_outputs_and_routes(lib, monkeypatch, capfd, rows, cols):
     """Each subset of the outputs has the bits of the full call; dx alone needs no workspace; more
     rows than CUs, outputs over inputs and forced tilings take the other kernels."""
