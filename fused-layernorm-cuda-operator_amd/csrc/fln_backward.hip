@@ -1684,7 +1684,10 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
   }
   p.stat_splits = static_cast<int>(splits);
   if (have_workspace) {
-    const size_t need = (static_cast<size_t>(part) +
+    // A call that needs no partial rows counts one block row of them all the same: what a fixed
+    // scratch refuses depends on the sizes alone, not on the route.
+    const size_t rows_needed = dgamma || dbeta ? static_cast<size_t>(2 * geo.blocks * ld) : 0;
+    const size_t need = (rows_needed +
                          (geo.two_pass ? 2 * static_cast<size_t>(p.rows * splits) : 0)) *
                         sizeof(float);
     if (need > workspace_bytes) return FLN_ERR_TOO_LARGE;

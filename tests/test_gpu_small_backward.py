@@ -104,3 +104,19 @@ def test_small_backward_outputs_and_routes(lib, monkeypatch, capfd, rows, cols):
     monkeypatch.delenv("FLN_BWD_SMALL_ROWS")
     capi.reload_tuning()
     assert not off
+
+
+@pytest.mark.parametrize("rows,cols,fits", [(1, 4194000, True), (1, 4194305, False),
+                                            (4, 4194305, False)])
+def test_one_block_row_keeps_the_scratch_limit(lib, rows, cols, fits):
+    """fln_layernorm_backward_noalloc holds 32 MiB: two fp32 rows of 4194304 columns, less the row
+    statistics, also where the column pass writes dgamma and dbeta itself."""
+    x = torch.randn(rows, cols, device="cuda")
+    mean, rstd = torch.zeros(rows, device="cuda"), torch.ones(rows, device="cuda")
+    dx, dg, db = torch.empty_like(x), torch.empty(cols, device="cuda"), torch.empty(cols,
+                                                                                  device="cuda")
+    p = capi.ptr
+    rc = lib.fln_layernorm_backward_noalloc(p(x), p(x), p(mean), p(rstd), None, None, p(dx), p(dg),
+                                            p(db), rows, cols, capi.F32, capi.F32, capi.stream())
+    torch.cuda.synchronize()
+    assert rc == (0 if fits else capi.ERR_TOO_LARGE)
