@@ -14,7 +14,7 @@
 // Both roles take unaligned vectors (RaggedRow), so any width of at least one vector runs here.
 //
 // Taken for at most one row per CU.  Backward calls, us, before -> here: fp32 32 x 768 6.4 -> 3.6, 128
-// x 768 6.9 -> 4.1, 256 x 768 7.7 -> 4.7, 256 x 16384 27.4 -> 18.2, 256 x 32768 36.8 -> 36.5; bf16 64 x
+// x 768 6.9 -> 3.8, 256 x 768 7.7 -> 4.7, 256 x 16384 27.4 -> 18.2, 256 x 32768 36.8 -> 36.5; bf16 64 x
 // 4096 8.1 -> 4.3, 256 x 1024 8.4 -> 4.8, 256 x 8192 19.5 -> 8.1, 200 x 12288 19.9 -> 7.6, 100 x 40000
 // 25.3 -> 14.7, 1 x 32768 11.5 -> 6.7; erf GELU 64 x 4096 9.5 -> 8.0, 100 x 30000
 // 32.3 -> 15.2; residual gradient 200 x 50000 41.1 -> 28.2.  More rows amortize the two stages'
