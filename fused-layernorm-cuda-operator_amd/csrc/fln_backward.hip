@@ -1660,6 +1660,7 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
   // workspace bound (fln_backward_workspace_bytes, not the size passed, so that the split and
   // with it the summation order never depend on the caller's workspace) leaves after the
   // partials.
+  const int64_t bound = 2 * workspace_partial_rows(p.rows) * ld + 2 * p.rows;
   int64_t splits = 1;
   const int64_t nvec = (p.cols + geo.vec - 1) / geo.vec;
   p.stat_chunk = nvec;
@@ -1674,7 +1675,6 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
     const int64_t steps = (nvec + step - 1) / step;
     splits = forced > 0 ? forced : (items + p.rows - 1) / p.rows;
     if (splits > kMaxStatSplits) splits = kMaxStatSplits;
-    const int64_t bound = 2 * workspace_partial_rows(p.rows) * ld + 2 * p.rows;
     const int64_t room = (bound - part) / (2 * p.rows);
     if (splits > room) splits = room;
     if (splits > steps) splits = steps;
@@ -1684,13 +1684,18 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
   }
   p.stat_splits = static_cast<int>(splits);
   if (have_workspace) {
-    // A call that needs no partial rows counts one block row of them all the same: what a fixed
-    // scratch refuses depends on the sizes alone, not on the route.
-    const size_t rows_needed = dgamma || dbeta ? static_cast<size_t>(2 * geo.blocks * ld) : 0;
-    const size_t need = (rows_needed +
-                         (geo.two_pass ? 2 * static_cast<size_t>(p.rows * splits) : 0)) *
-                        sizeof(float);
-    if (need > workspace_bytes) return FLN_ERR_TOO_LARGE;
+    const int64_t stats = geo.two_pass ? 2 * p.rows * splits : 0;
+    int64_t need = part + stats;
+    if (direct && (dgamma || dbeta)) {
+      // A call that needs no partial rows counts one block row of them all the same, and of its
+      // statistics no more than the bound leaves beside that (one row has 16 splits where the
+      // partial rows would be): what a fixed scratch refuses depends on the sizes alone, not on
+      // the route, and a workspace of the bound always holds the call.
+      const int64_t left = bound - 2 * ld;
+      const int64_t counted = 2 * ld + (stats < left ? stats : left);
+      if (counted > need) need = counted;
+    }
+    if (static_cast<size_t>(need) * sizeof(float) > workspace_bytes) return FLN_ERR_TOO_LARGE;
   }
   if ((dgamma || dbeta) && dparam_dtype != FLN_F32 && dparam_dtype != FLN_BF16 &&
       dparam_dtype != FLN_F16)
