@@ -825,7 +825,8 @@ __global__ __launch_bounds__(kFwdLdsThreads) void fwd_lds_kernel(const FwdParams
 //     count (mean_t - mean)^2 -- two block reductions in a fixed order, so the statistics are
 //     bitwise reproducible and need no E[x^2] - mean^2 cancellation.  RMSNorm sums squares;
 //   pass 2, fp8 with a per-row scale only: the row maximum of the outputs;
-//   last pass: outputs (and, with a residual, h = x + r written during pass 1).
+//   last pass: outputs (and, with a residual, h = x + r written during pass 1; the later passes
+//     form x + r again, or read h where it lies over an input: INPLACE).
 // x (and the residual) are read once per pass, the passes walking the row in alternate
 // directions so that each starts on the lines the previous one read last, which are still in L2
 // (the last pass loads non-temporal).  Most of a later pass still comes from HBM: at 131072
@@ -834,13 +835,16 @@ __global__ __launch_bounds__(kFwdLdsThreads) void fwd_lds_kernel(const FwdParams
 constexpr int kFwdWideThreads = 1024;
 constexpr int kFwdWideStepBytes = 64;  // bytes of the row per thread and step (4 vectors)
 
-// OWN (ragged rows with an output over an input): the row's last vector is written by element.
-template <class T, int FP8, bool RES, int GELU, int VEC, bool RAGGED, bool OWN = false>
+// INPLACE: an output lies over an input (h over x or r; ragged rows also y over x or r).  With a
+// residual the passes after the first read the stored h where there is one: the inputs that they
+// would add again may hold h by then.  A ragged row's last vector is written by element.
+template <class T, int FP8, bool RES, int GELU, int VEC, bool RAGGED, bool INPLACE = false>
 __global__ __launch_bounds__(kFwdWideThreads)
 // Ragged 16-bit LayerNorm / RMSNorm took 66 VGPRs, one block per CU: 2048 x 24001 80.4 us against 69.9
 // with two.
-__attribute__((amdgpu_waves_per_eu(RAGGED && !RES && !OWN && GELU == 0 && FP8 == 0 ? 8 : 4)))
+__attribute__((amdgpu_waves_per_eu(RAGGED && !RES && !INPLACE && GELU == 0 && FP8 == 0 ? 8 : 4)))
 void fwd_wide_kernel(const FwdParams p) {
+  constexpr bool OWN = INPLACE && RAGGED;
   constexpr int kT = kFwdWideThreads;
   constexpr int kW = kT / kWave;
   constexpr int U = kFwdWideStepBytes / (VEC * static_cast<int>(sizeof(T)));
@@ -879,10 +883,20 @@ void fwd_wide_kernel(const FwdParams p) {
     float(*slots)[kW + 16] = red[parity];
     const rsrc_t xq = make_rsrc(X + row * N, row_bytes);
     const rsrc_t rq = make_rsrc(RES ? R + row * N : nullptr, row_bytes);
+    const rsrc_t hr = make_rsrc(RES && p.h ? static_cast<T*>(p.h) + row * N : nullptr,
+                                row_bytes);
     // Step `base`: vectors base + t + kT u of the row (zeros past the row); with a residual,
-    // h = x + r rounded to T, as every pass recomputes it.
-    auto load_step = [&](uint32_t base, P (&hv)[U], auto pol) {
+    // h = x + r rounded to T, as every pass recomputes it, or (stored, INPLACE) reads it back.
+    auto load_step = [&](uint32_t base, P (&hv)[U], auto pol, bool stored = true) {
       constexpr int POL = decltype(pol)::value;
+      if constexpr (INPLACE && RES) {
+        if (stored && p.h != nullptr) {  // uniform
+#pragma unroll
+          for (int u = 0; u < U; ++u) hv[u] = buf_load_at<P, POL>(hr, off(base + t + kT * u));
+          return;
+        }
+      }
+      (void)stored;
       P rv[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -902,13 +916,11 @@ void fwd_wide_kernel(const FwdParams p) {
     using Last = std::integral_constant<int, kStream>;
 
     // Pass 1: statistics (and h).
-    const rsrc_t hr = make_rsrc(RES && p.h ? static_cast<T*>(p.h) + row * N : nullptr,
-                                row_bytes);
     float mean = 0.0f, rstd;
     float cnt = 0.0f, mu = 0.0f, m2 = 0.0f;  // this thread's elements: count, mean, M2
     for (uint32_t base = 0; base < nvec; base += kT * U) {
       P hv[U];
-      load_step(base, hv, Keep{});
+      load_step(base, hv, Keep{}, false);
       // A ragged row's last step: its last vector counts only its own elements.
       const bool tail = RAGGED && base + kT * U > rag.nfull;  // uniform
       if constexpr (RES) {
@@ -975,6 +987,9 @@ void fwd_wide_kernel(const FwdParams p) {
         cnt = nn;
       }
     }
+    // The barrier of the reduction below separates the stores of h from the loads of it; it does
+    // not wait for them by itself (vmcnt(0), the other counters as they are).
+    if constexpr (INPLACE && RES) __builtin_amdgcn_s_waitcnt(0x0f70);
     if (p.rms) {
       const float q = row_allreduce<SumOp>(m2, slots[0], kW, 0, wave, lane);
       rstd = __builtin_amdgcn_rsqf(q * inv_n + p.eps);  // v_rsq_f32, 1 ulp
@@ -1117,22 +1132,26 @@ __global__ __launch_bounds__(1024) void fwd_loop_kernel(const FwdParams p) {
   const T* b = static_cast<const T*>(p.beta);
   for (int64_t row = blockIdx.x; row < p.rows; row += gridDim.x) {
     const int64_t base = row * N;
-    auto in = [&](int64_t j) -> A {
+    auto sum_in = [&](int64_t j) -> A {
       if (r) return static_cast<A>(static_cast<T>(static_cast<A>(x[base + j]) +
                                                   static_cast<A>(r[base + j])));
       return static_cast<A>(x[base + j]);
     };
+    // After the first pass, h where it is stored (each thread reads back its own elements): it may
+    // lie over x or r.
+    auto in = [&](int64_t j) -> A { return h ? static_cast<A>(h[base + j]) : sum_in(j); };
     A mean = 0;
     if (!p.rms) {
       A s = 0;
       for (int64_t j = threadIdx.x; j < N; j += blockDim.x) {
-        const A v = in(j);
+        const A v = sum_in(j);
         if (h) h[base + j] = static_cast<T>(v);
         s += v;
       }
       mean = block_allreduce<A, false>(s, red[0]) / static_cast<A>(N);
     } else if (h) {
-      for (int64_t j = threadIdx.x; j < N; j += blockDim.x) h[base + j] = static_cast<T>(in(j));
+      for (int64_t j = threadIdx.x; j < N; j += blockDim.x)
+        h[base + j] = static_cast<T>(sum_in(j));
     }
     A q = 0;
     for (int64_t j = threadIdx.x; j < N; j += blockDim.x) {
@@ -1810,11 +1829,17 @@ int launch_wide(const FwdParams& p, hipStream_t s) {
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kFwdWideThreads), 0, s, p);
     return static_cast<int>(hipGetLastError());
   };
+  const int64_t bytes = p.rows * p.cols * static_cast<int64_t>(sizeof(T));
+  auto over_input = [&](const void* out) {
+    return overlaps(out, bytes, p.x, bytes) || overlaps(out, bytes, p.res, bytes);
+  };
+  // y over an input is written where it was read, by the same thread, but for the elements that a
+  // ragged row's last vectors share (fp8 codes over an input never were in place).
+  const bool y_over = RAGGED && FP8 == 0 && over_input(p.y);
+  if (p.res && (y_over || over_input(p.h)))
+    return launch(fwd_wide_kernel<T, FP8, true, 0, VEC, RAGGED, true>);
   if constexpr (RAGGED && FP8 == 0) {
-    const int64_t bytes = p.rows * p.cols * static_cast<int64_t>(sizeof(T));
-    if (overlaps(p.y, bytes, p.x, bytes) || overlaps(p.y, bytes, p.res, bytes) ||
-        overlaps(p.h, bytes, p.x, bytes) || overlaps(p.h, bytes, p.res, bytes)) {
-      if (p.res) return launch(fwd_wide_kernel<T, 0, true, 0, VEC, true, true>);
+    if (y_over) {
       if (p.gelu == FLN_GELU_ERF) return launch(fwd_wide_kernel<T, 0, false, 1, VEC, true, true>);
       if (p.gelu == FLN_GELU_TANH) return launch(fwd_wide_kernel<T, 0, false, 2, VEC, true, true>);
       return launch(fwd_wide_kernel<T, 0, false, 0, VEC, true, true>);

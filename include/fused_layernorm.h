@@ -8,6 +8,11 @@
  * arguments (detected before anything is launched), or a nonzero hipError_t value from the
  * launch.  fln_error_string() turns a code into text.
  *
+ * In place: y (in the I/O type) and h may be x and the residual themselves, one each, and dx may be
+ * dy, x or dres.  Another kernel may take such a call than separate buffers take, so the results
+ * are equal up to the rounding of another summation order.  Outputs that overlap an input in any
+ * other way, fp8 codes over an input included, are not supported.
+ *
  * Each entry point names the reference interface it replaces (paths relative to the
  * JonSnow1807/Fused-LayerNorm-CUDA-Operator tree).
  */
