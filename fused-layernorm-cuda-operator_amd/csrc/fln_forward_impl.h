@@ -1817,18 +1817,24 @@ int launch_split(FwdParams p, hipStream_t s) {
              fwd_split_out_kernel<T, FP8, false, 0, VEC, true>);
 }
 
+// KERNEL: a template argument, so that each kernel has an occupancy cache of its own (they share one
+// type; some fit a CU twice and some once).
+template <void (*KERNEL)(FwdParams)>
+int launch_wide_kernel(const FwdParams& p, hipStream_t s) {
+  static std::atomic<int> occupancy_cache[64];  // per device
+  int64_t grid = resident_blocks(KERNEL, kFwdWideThreads, occupancy_cache);
+  const int forced = tuning().fwd_grid_mult;  // FLN_FWD_GRID_MULT: blocks per CU
+  if (forced > 0 && grid > forced * device_cu_count()) grid = forced * device_cu_count();
+  if (grid > p.rows) grid = p.rows;
+  if (grid > kMaxGrid) grid = kMaxGrid;
+  if (tuning().debug_geometry > 1)
+    fprintf(stderr, "fln wide: blocks=%lld\n", static_cast<long long>(grid));
+  hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(kFwdWideThreads), 0, s, p);
+  return static_cast<int>(hipGetLastError());
+}
+
 template <class T, int FP8, int VEC, bool RAGGED>
 int launch_wide(const FwdParams& p, hipStream_t s) {
-  auto launch = [&](auto kernel) {
-    static std::atomic<int> occupancy_cache[64];  // per instantiation, per device
-    int64_t grid = resident_blocks(kernel, kFwdWideThreads, occupancy_cache);
-    const int forced = tuning().fwd_grid_mult;  // FLN_FWD_GRID_MULT: blocks per CU
-    if (forced > 0 && grid > forced * device_cu_count()) grid = forced * device_cu_count();
-    if (grid > p.rows) grid = p.rows;
-    if (grid > kMaxGrid) grid = kMaxGrid;
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kFwdWideThreads), 0, s, p);
-    return static_cast<int>(hipGetLastError());
-  };
   const int64_t bytes = p.rows * p.cols * static_cast<int64_t>(sizeof(T));
   auto over_input = [&](const void* out) {
     return overlaps(out, bytes, p.x, bytes) || overlaps(out, bytes, p.res, bytes);
@@ -1837,20 +1843,24 @@ int launch_wide(const FwdParams& p, hipStream_t s) {
   // ragged row's last vectors share (fp8 codes over an input never were in place).
   const bool y_over = RAGGED && FP8 == 0 && over_input(p.y);
   if (p.res && (y_over || over_input(p.h)))
-    return launch(fwd_wide_kernel<T, FP8, true, 0, VEC, RAGGED, true>);
+    return launch_wide_kernel<fwd_wide_kernel<T, FP8, true, 0, VEC, RAGGED, true>>(p, s);
   if constexpr (RAGGED && FP8 == 0) {
     if (y_over) {
-      if (p.gelu == FLN_GELU_ERF) return launch(fwd_wide_kernel<T, 0, false, 1, VEC, true, true>);
-      if (p.gelu == FLN_GELU_TANH) return launch(fwd_wide_kernel<T, 0, false, 2, VEC, true, true>);
-      return launch(fwd_wide_kernel<T, 0, false, 0, VEC, true, true>);
+      if (p.gelu == FLN_GELU_ERF)
+        return launch_wide_kernel<fwd_wide_kernel<T, 0, false, 1, VEC, true, true>>(p, s);
+      if (p.gelu == FLN_GELU_TANH)
+        return launch_wide_kernel<fwd_wide_kernel<T, 0, false, 2, VEC, true, true>>(p, s);
+      return launch_wide_kernel<fwd_wide_kernel<T, 0, false, 0, VEC, true, true>>(p, s);
     }
   }
-  if (p.res) return launch(fwd_wide_kernel<T, FP8, true, 0, VEC, RAGGED>);
+  if (p.res) return launch_wide_kernel<fwd_wide_kernel<T, FP8, true, 0, VEC, RAGGED>>(p, s);
   if constexpr (FP8 == 0) {
-    if (p.gelu == FLN_GELU_ERF) return launch(fwd_wide_kernel<T, 0, false, 1, VEC, RAGGED>);
-    if (p.gelu == FLN_GELU_TANH) return launch(fwd_wide_kernel<T, 0, false, 2, VEC, RAGGED>);
+    if (p.gelu == FLN_GELU_ERF)
+      return launch_wide_kernel<fwd_wide_kernel<T, 0, false, 1, VEC, RAGGED>>(p, s);
+    if (p.gelu == FLN_GELU_TANH)
+      return launch_wide_kernel<fwd_wide_kernel<T, 0, false, 2, VEC, RAGGED>>(p, s);
   }
-  return launch(fwd_wide_kernel<T, FP8, false, 0, VEC, RAGGED>);
+  return launch_wide_kernel<fwd_wide_kernel<T, FP8, false, 0, VEC, RAGGED>>(p, s);
 }
 
 template <class T, class A, int FP8>

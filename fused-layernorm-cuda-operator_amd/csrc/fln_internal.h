@@ -125,7 +125,7 @@ struct Tuning {
   int fwd_epl;         // FLN_FWD_EPL: forward elements per lane for rows of up to 4 waves
   int fwd_wpr;         // FLN_FWD_WPR: forward waves per row
   int fwd_grid_mult;   // FLN_FWD_GRID_MULT: forward grid = this many blocks per CU
-  int debug_geometry;  // FLN_DEBUG_GEOMETRY: one stderr line per forward launch
+  int debug_geometry;  // FLN_DEBUG_GEOMETRY: one stderr line per launch (2: streamed grids as well)
   int fwd_no_lds;      // FLN_FWD_NO_LDS: never the LDS-staged forward
   int fwd_no_wide;     // FLN_FWD_NO_WIDE: the looped forward instead of the streamed wide-row one
   int fwd_no_split;    // FLN_FWD_NO_SPLIT: never the few-row split forward

@@ -104,3 +104,28 @@ def test_ragged_in_place(lib, dtype, rows, cols):
     for a, c in zip(*outs):  # another route may sum in another order: one rounding of the type
         scale = c.float().abs().max()
         assert (a.float() - c.float()).abs().max() <= (ulp if a.dtype == dtype else 1e-5) * scale
+
+
+def test_streamed_grids_do_not_depend_on_the_calls_before(lib, monkeypatch, capfd):
+    """The grid of a streamed forward is what its own kernel's occupancy gives, whichever flavour ran
+    first: a ragged bf16 LayerNorm fits a CU twice, residual + LayerNorm (over 64 VGPRs) once."""
+    cols, p, st = 20001, capi.ptr, capi.stream()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rows = 2 * cus
+    x = torch.randn(rows, cols, device="cuda", dtype=torch.bfloat16)
+    y, h = torch.empty_like(x), torch.empty_like(x)
+    monkeypatch.setenv("FLN_DEBUG_GEOMETRY", "2")
+    capi.reload_tuning()
+    grids = []
+    for _ in range(2):
+        for residual in (True, False):
+            capfd.readouterr()
+            if residual:
+                rc = lib.fln_add_layernorm_forward(p(x), p(x), None, None, p(h), p(y), None, None,
+                                                   rows, cols, capi.BF16, 1e-5, st)
+            else:
+                rc = lib.fln_layernorm(p(x), None, None, p(y), rows, cols, capi.BF16, 1e-5, st)
+            capi.check(rc)
+            torch.cuda.synchronize()
+            grids.append(int(capfd.readouterr().err.split("fln wide: blocks=")[1].split()[0]))
+    assert grids == [cus, 2 * cus] * 2
