@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/dynamo/compiled_autograd.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
 #include <array>
@@ -554,6 +555,171 @@ std::string get_performance_hints(int batch_size, int hidden_size) {
 }
 
 // ------------------------------------------------------------------------------------------
+// Backward of the autograd nodes below, from their saved tensors.
+// ------------------------------------------------------------------------------------------
+using torch::autograd::variable_list;
+enum NormKind { kLayerNorm = 0, kRmsNorm = 1, kLayerNormGelu = 2, kAddLayerNorm = 3, kAddRmsNorm = 4 };
+
+// Whether a call on these tensors may pass the dispatcher by: ordinary GPU tensors, nothing that
+// watches or rewrites operator calls (dispatch modes, tracing, functorch transforms, subclasses),
+// no forward-mode tangents.
+bool plain_call(std::initializer_list<const Tensor*> tensors) {
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing() ||
+      c10::impl::tls_local_dispatch_key_set().included_.has(
+          c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+    return false;
+  constexpr c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::Functionalize,
+                                         c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::FuncTorchBatched,
+                                         c10::DispatchKey::Batched, c10::DispatchKey::Conjugate,
+                                         c10::DispatchKey::Negative});
+  for (const Tensor* t : tensors) {
+    if (t == nullptr || !t->defined()) continue;
+    if (!t->is_cuda() || t->layout() != at::kStrided || t->key_set().has_any(special) ||
+        t->_fw_grad(0).defined())
+      return false;
+  }
+  return true;
+}
+
+// The [rows, n] form of a contiguous tensor, and a 1-D form of a parameter.
+Tensor as_rows(const Tensor& t, int64_t n) {
+  return t.dim() == 2 && t.size(1) == n ? t : t.view({t.numel() / n, n});
+}
+OptT as_param(const OptT& p) {
+  return has(p) && p->dim() != 1 ? OptT(p->reshape({-1})) : p;
+}
+
+// A registered backward operator by name, or the function itself where nothing watches.
+template <class Fn, class... Args>
+auto call_operator(bool direct, const char* op, Fn* fn, Args&&... args) {
+  if (direct) return fn(std::forward<Args>(args)...);
+  return c10::Dispatcher::singleton()
+      .findSchemaOrThrow(op, "")
+      .template typed<Fn>()
+      .call(std::forward<Args>(args)...);
+}
+
+// Gradients of the input (for `add` kinds also of the residual), weight and bias where `needs` asks
+// for them.  gy: the gradient of the norm's output; gh: of the residual sum.  rows: the normalized
+// tensor (the input, or the residual sum), whose last dimensions hold n elements.
+struct NormGrads {
+  Tensor dx, dw, db;
+};
+NormGrads norm_backward(NormKind kind, int64_t n, const std::string& approximate, Tensor gy,
+                        const Tensor& gh, const Tensor& rows, const OptT& w, const OptT& b,
+                        const Tensor& mean, const Tensor& rstd, std::array<bool, 3> needs) {
+  // Differentiating this backward, or a mode or subclass that looks on: the operators.
+  const bool direct =
+      !c10::GradMode::is_enabled() &&
+      plain_call({&rows, &rstd, &mean, w ? &*w : nullptr, b ? &*b : nullptr, &gy, &gh});
+  std::optional<at::AutoDispatchBelowADInplaceOrView> below;
+  if (direct) below.emplace();
+  // Sizes may be symbolic where the operators are taken.
+  auto flat = [&](const Tensor& t) { return direct ? as_rows(t, n) : t.view({-1, n}); };
+  auto shaped = [&](const Tensor& t, const Tensor& as) {
+    return direct && t.sizes() == as.sizes() ? t : t.view_as(as);
+  };
+  if (!gy.defined()) gy = at::zeros_like(rows);
+  const Tensor x2 = flat(rows), dy2 = flat(gy.contiguous());
+  const OptT extra = gh.defined() ? OptT(flat(gh.contiguous())) : std::nullopt;
+  const OptT w1 = as_param(w), b1 = as_param(b);
+  NormGrads g;
+  if (kind == kRmsNorm || kind == kAddRmsNorm) {
+    std::tie(g.dx, g.dw) =
+        call_operator(direct, "fused_layernorm::rms_norm_bwd", &rms_norm_bwd, dy2, x2, rstd, w1,
+                      std::array<bool, 2>{needs[0], needs[1]}, extra);
+  } else if (kind == kLayerNormGelu) {
+    std::tie(g.dx, g.dw, g.db) =
+        call_operator(direct, "fused_layernorm::layer_norm_gelu_bwd", &layer_norm_gelu_bwd, dy2,
+                      x2, mean, rstd, w1, b1, approximate, needs);
+  } else {
+    std::tie(g.dx, g.dw, g.db) =
+        call_operator(direct, "fused_layernorm::layer_norm_bwd", &layer_norm_bwd, dy2, x2, mean,
+                      rstd, w1, b1, needs, extra);
+  }
+  g.dx = needs[0] ? shaped(g.dx, rows) : Tensor();
+  g.dw = needs[1] ? shaped(g.dw, *w) : Tensor();
+  g.db = needs[2] ? shaped(g.db, *b) : Tensor();
+  return g;
+}
+
+// Compiled autograd captures a backward as a graph: a node hands over what it saved
+// (compiled_args), and where the graph is built its place is taken by a call of a function of the
+// incoming gradients and those values (apply_with_saved), here captured_backward.
+using torch::dynamo::autograd::CompiledNodeArgs;
+using torch::dynamo::autograd::PackedArgs;
+using torch::dynamo::autograd::SwapSavedVariables;
+
+variable_list captured_backward(const variable_list& grads,
+                                const torch::autograd::ivalue_list& values) {
+  PackedArgs args(values);
+  const NormKind kind = static_cast<NormKind>(args.unpack<int64_t>());
+  const int64_t n = args.unpack<int64_t>();
+  const int64_t edges = args.unpack<int64_t>();
+  const std::string approximate = args.unpack<std::string>();
+  const bool has_w = args.unpack<bool>(), has_b = args.unpack<bool>();
+  const std::array<bool, 4> needs = args.unpack<std::array<bool, 4>>();  // x, residual, w, b
+  const variable_list saved = args.unpack<variable_list>();  // rows, w, b, rstd, mean: the present
+  const bool add = kind == kAddLayerNorm || kind == kAddRmsNorm;
+  const bool rms = kind == kRmsNorm || kind == kAddRmsNorm;
+  size_t i = 0;
+  const Tensor rows = saved[i++];
+  const OptT w = has_w ? OptT(saved[i++]) : std::nullopt;
+  const OptT b = has_b ? OptT(saved[i++]) : std::nullopt;
+  const Tensor rstd = saved[i++], mean = rms ? Tensor() : saved[i++];
+  const Tensor gh = add ? grads[1] : Tensor();
+  variable_list out(4);
+  const std::array<bool, 3> wanted{needs[0] || (add && needs[1]), has_w && needs[2],
+                                   has_b && needs[3]};
+  if ((grads[0].defined() || gh.defined()) && (wanted[0] || wanted[1] || wanted[2])) {
+    const NormGrads g =
+        norm_backward(kind, n, approximate, grads[0], gh, rows, w, b, mean, rstd, wanted);
+    if (needs[0]) out[0] = g.dx;
+    if (add && needs[1]) out[1] = g.dx;
+    out[2] = g.dw;
+    out[3] = g.db;
+  }
+  if (edges < 4) out.erase(out.begin() + 1);  // the one-dimensional nodes: no residual,
+  if (edges < 3) out.pop_back();              // RMSNorm's no bias
+  return out;
+}
+
+// apply_with_saved of a node: `vars` are its saved variables (all of compiled_args'), `saved` the
+// list for captured_backward while they hold the graph's values.
+template <class Saved>
+variable_list capture_backward(torch::autograd::Node& node, SwapSavedVariables& swap,
+                               const variable_list& grads,
+                               std::initializer_list<torch::autograd::SavedVariable*> vars,
+                               NormKind kind, int64_t n, const std::string& approximate,
+                               bool has_w, bool has_b, std::array<bool, 4> needs, Saved&& saved) {
+  namespace ca = torch::dynamo::autograd;
+  for (auto* v : vars) swap.before(*v);
+  PackedArgs args;
+  args.pack(static_cast<int64_t>(kind));
+  args.pack(n);
+  args.pack(static_cast<int64_t>(node.num_outputs()));
+  args.pack(approximate);
+  args.pack(has_w);
+  args.pack(has_b);
+  args.pack(needs);
+  args.pack(variable_list(saved()));
+  std::vector<at::TypePtr> types;
+  for (const at::IValue& v : args.vec()) types.push_back(v.type());
+  const auto& compiler = ca::getPyCompilerInterface();
+  const std::string fn = compiler->bind_function(swap.get_py_compiler(), node.name(),
+                                                 &captured_backward, types,
+                                                 /*is_custom_function=*/true,
+                                                 /*is_traceable=*/true);
+  variable_list out = compiler->call_function(
+      swap.get_py_compiler(), "apply_functional", fn, grads, args.vec(),
+      ca::IValuePacker<std::vector<std::optional<torch::autograd::InputMetadata>>>::pack(
+          ca::get_input_metadata(node.next_edges())));
+  for (auto* v : vars) swap.after(*v);
+  return out;
+}
+
+// ------------------------------------------------------------------------------------------
 // LayerNorm with autograd in C++: the eager path of FusedLayerNorm / fused_layer_norm.  A
 // Python torch.autograd.Function plus an operator call cost ~10 us per forward on the host (the
 // GPU work at BERT shapes is ~3 us).  Here the output gets a graph node of its own, built the way
@@ -566,9 +732,10 @@ std::string get_performance_hints(int batch_size, int hidden_size) {
 // ------------------------------------------------------------------------------------------
 struct FusedLayerNormBackward : public torch::autograd::Node {
   torch::autograd::SavedVariable x_, w_, b_, stats_;
+  int64_t n = 0;
   bool has_w = false, has_b = false;
 
-  torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+  variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     const Tensor x = x_.unpack(), stats = stats_.unpack();
     const OptT w = has_w ? OptT(w_.unpack()) : std::nullopt;
@@ -581,6 +748,28 @@ struct FusedLayerNormBackward : public torch::autograd::Node {
     auto r = layer_norm_bwd(dy, x, stats[0], stats[1], w, b, mask, std::nullopt);
     return {mask[0] ? std::get<0>(r) : Tensor(), mask[1] ? std::get<1>(r) : Tensor(),
             mask[2] ? std::get<2>(r) : Tensor()};
+  }
+  void compiled_args(CompiledNodeArgs& args) const override {
+    for (const auto* v : {&x_, &w_, &b_, &stats_}) args.collect(*v, false);
+    args.collect(n);
+    args.collect(has_w);
+    args.collect(has_b);
+  }
+  variable_list apply_with_saved(const variable_list& grads, SwapSavedVariables& swap) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    return capture_backward(*this, swap, grads, {&x_, &w_, &b_, &stats_}, kLayerNorm, n, "", has_w,
+                            has_b,
+                            {task_should_compute_output(0), false, task_should_compute_output(1),
+                             task_should_compute_output(2)},
+                            [&] {
+                              variable_list saved{x_.unpack()};
+                              if (has_w) saved.push_back(w_.unpack());
+                              if (has_b) saved.push_back(b_.unpack());
+                              const Tensor stats = stats_.unpack();
+                              saved.push_back(stats[1]);
+                              saved.push_back(stats[0]);
+                              return saved;
+                            });
   }
   std::string name() const override { return "FusedLayerNormBackward"; }
   void release_variables() override {
@@ -620,6 +809,7 @@ Tensor layer_norm_autograd(const Tensor& input, int64_t normalized, const OptT& 
         x, has(weight) ? *weight : Tensor(), has(bias) ? *bias : Tensor()));
     node->x_ = torch::autograd::SavedVariable(x, false);
     node->stats_ = torch::autograd::SavedVariable(stats, false);
+    node->n = normalized;
     node->has_w = has(weight);
     node->has_b = has(bias);
     if (node->has_w) node->w_ = torch::autograd::SavedVariable(*weight, false);
@@ -633,9 +823,10 @@ Tensor layer_norm_autograd(const Tensor& input, int64_t normalized, const OptT& 
 // layer_norm_autograd (saves input, weight, rstd).
 struct FusedRMSNormBackward : public torch::autograd::Node {
   torch::autograd::SavedVariable x_, w_, rstd_;
+  int64_t n = 0;
   bool has_w = false;
 
-  torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+  variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     const Tensor x = x_.unpack(), rstd = rstd_.unpack();
     const OptT w = has_w ? OptT(w_.unpack()) : std::nullopt;
@@ -645,6 +836,23 @@ struct FusedRMSNormBackward : public torch::autograd::Node {
     const Tensor dy = grads[0].is_contiguous() ? grads[0] : grads[0].contiguous();
     auto r = rms_norm_bwd(dy, x, rstd, w, mask, std::nullopt);
     return {mask[0] ? std::get<0>(r) : Tensor(), mask[1] ? std::get<1>(r) : Tensor()};
+  }
+  void compiled_args(CompiledNodeArgs& args) const override {
+    for (const auto* v : {&x_, &w_, &rstd_}) args.collect(*v, false);
+    args.collect(n);
+    args.collect(has_w);
+  }
+  variable_list apply_with_saved(const variable_list& grads, SwapSavedVariables& swap) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    return capture_backward(*this, swap, grads, {&x_, &w_, &rstd_}, kRmsNorm, n, "", has_w, false,
+                            {task_should_compute_output(0), false, task_should_compute_output(1),
+                             false},
+                            [&] {
+                              variable_list saved{x_.unpack()};
+                              if (has_w) saved.push_back(w_.unpack());
+                              saved.push_back(rstd_.unpack());
+                              return saved;
+                            });
   }
   std::string name() const override { return "FusedRMSNormBackward"; }
   void release_variables() override {
@@ -671,6 +879,7 @@ Tensor rms_norm_autograd(const Tensor& input, int64_t normalized, const OptT& we
         torch::autograd::collect_next_edges(x, has(weight) ? *weight : Tensor()));
     node->x_ = torch::autograd::SavedVariable(x, false);
     node->rstd_ = torch::autograd::SavedVariable(std::get<1>(r), false);
+    node->n = normalized;
     node->has_w = has(weight);
     if (node->has_w) node->w_ = torch::autograd::SavedVariable(*weight, false);
     torch::autograd::set_history(y, node);
@@ -687,37 +896,6 @@ Tensor rms_norm_autograd(const Tensor& input, int64_t normalized, const OptT& we
 // Here one node holds what the operators' formulas save (the normalized rows, weight, bias, mean,
 // rstd) and its backward calls the same functions, so outputs and gradients are the same bits.
 // ------------------------------------------------------------------------------------------
-enum NormKind { kLayerNorm = 0, kRmsNorm = 1, kLayerNormGelu = 2, kAddLayerNorm = 3, kAddRmsNorm = 4 };
-
-// Whether a call on these tensors may pass the dispatcher by: ordinary GPU tensors, nothing that
-// watches or rewrites operator calls (dispatch modes, tracing, functorch transforms, subclasses),
-// no forward-mode tangents.
-bool plain_call(std::initializer_list<const Tensor*> tensors) {
-  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing() ||
-      c10::impl::tls_local_dispatch_key_set().included_.has(
-          c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
-    return false;
-  constexpr c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::Functionalize,
-                                         c10::DispatchKey::FuncTorchGradWrapper,
-                                         c10::DispatchKey::FuncTorchBatched,
-                                         c10::DispatchKey::Batched, c10::DispatchKey::Conjugate,
-                                         c10::DispatchKey::Negative});
-  for (const Tensor* t : tensors) {
-    if (t == nullptr || !t->defined()) continue;
-    if (!t->is_cuda() || t->layout() != at::kStrided || t->key_set().has_any(special) ||
-        t->_fw_grad(0).defined())
-      return false;
-  }
-  return true;
-}
-
-// The [rows, n] form of a contiguous tensor, and a 1-D form of a parameter.
-Tensor as_rows(const Tensor& t, int64_t n) {
-  return t.dim() == 2 && t.size(1) == n ? t : t.view({t.numel() / n, n});
-}
-OptT as_param(const OptT& p) {
-  return has(p) && p->dim() != 1 ? OptT(p->reshape({-1})) : p;
-}
 
 struct FusedNormBackward : public torch::autograd::Node {
   torch::autograd::SavedVariable rows_, w_, b_, mean_, rstd_;  // rows_: the input, or h
@@ -726,21 +904,11 @@ struct FusedNormBackward : public torch::autograd::Node {
   std::string approximate;
   bool has_w = false, has_b = false;
 
-  // A registered backward operator by name, or the function itself where nothing watches.
-  template <class Fn, class... Args>
-  static auto call(bool direct, const char* op, Fn* fn, Args&&... args) {
-    if (direct) return fn(std::forward<Args>(args)...);
-    return c10::Dispatcher::singleton()
-        .findSchemaOrThrow(op, "")
-        .template typed<Fn>()
-        .call(std::forward<Args>(args)...);
-  }
-
-  torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+  variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     const bool add = kind == kAddLayerNorm || kind == kAddRmsNorm;
     const bool rms = kind == kRmsNorm || kind == kAddRmsNorm;
-    torch::autograd::variable_list out(4);
+    variable_list out(4);
     Tensor gy = grads[0], gh = add ? grads[1] : Tensor();
     const bool need_x = task_should_compute_output(0) || (add && task_should_compute_output(1));
     const bool need_w = has_w && task_should_compute_output(2);
@@ -750,38 +918,38 @@ struct FusedNormBackward : public torch::autograd::Node {
     const Tensor rstd = rstd_.unpack(), mean = rms ? Tensor() : mean_.unpack();
     const OptT w = has_w ? OptT(w_.unpack()) : std::nullopt;
     const OptT b = has_b ? OptT(b_.unpack()) : std::nullopt;
-    // Differentiating this backward, or a mode or subclass that looks on: the operators.
-    const bool direct =
-        !c10::GradMode::is_enabled() &&
-        plain_call({&rows, &rstd, &mean, w ? &*w : nullptr, b ? &*b : nullptr, &gy, &gh});
-    std::optional<at::AutoDispatchBelowADInplaceOrView> below;
-    if (direct) below.emplace();
-    if (!gy.defined()) gy = at::zeros_like(rows);
-    const Tensor x2 = as_rows(rows, n), dy2 = as_rows(gy.contiguous(), n);
-    const OptT extra = gh.defined() ? OptT(as_rows(gh.contiguous(), n)) : std::nullopt;
-    const OptT w1 = as_param(w), b1 = as_param(b);
-    Tensor dx, dw, db;
-    if (rms) {
-      std::tie(dx, dw) =
-          call(direct, "fused_layernorm::rms_norm_bwd", &rms_norm_bwd, dy2, x2, rstd, w1,
-               std::array<bool, 2>{need_x, need_w}, extra);
-    } else if (kind == kLayerNormGelu) {
-      std::tie(dx, dw, db) =
-          call(direct, "fused_layernorm::layer_norm_gelu_bwd", &layer_norm_gelu_bwd, dy2, x2,
-               mean, rstd, w1, b1, approximate, std::array<bool, 3>{need_x, need_w, need_b});
-    } else {
-      std::tie(dx, dw, db) =
-          call(direct, "fused_layernorm::layer_norm_bwd", &layer_norm_bwd, dy2, x2, mean, rstd,
-               w1, b1, std::array<bool, 3>{need_x, need_w, need_b}, extra);
-    }
-    if (need_x) {
-      if (dx.sizes() != rows.sizes()) dx = dx.view(rows.sizes());
-      if (task_should_compute_output(0)) out[0] = dx;
-      if (add && task_should_compute_output(1)) out[1] = dx;
-    }
-    if (need_w) out[2] = w->dim() == 1 ? dw : dw.view(w->sizes());
-    if (need_b) out[3] = b->dim() == 1 ? db : db.view(b->sizes());
+    NormGrads g = norm_backward(kind, n, approximate, gy, gh, rows, w, b, mean, rstd,
+                                {need_x, need_w, need_b});
+    if (task_should_compute_output(0)) out[0] = g.dx;
+    if (add && task_should_compute_output(1)) out[1] = g.dx;
+    out[2] = std::move(g.dw);
+    out[3] = std::move(g.db);
     return out;
+  }
+  void compiled_args(CompiledNodeArgs& args) const override {
+    args.collect(rows_, kind == kAddLayerNorm || kind == kAddRmsNorm);
+    for (const auto* v : {&w_, &b_, &mean_, &rstd_}) args.collect(*v, false);
+    args.collect(static_cast<int64_t>(kind));
+    args.collect(n);
+    args.collect(approximate);
+    args.collect(has_w);
+    args.collect(has_b);
+  }
+  variable_list apply_with_saved(const variable_list& grads, SwapSavedVariables& swap) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    return capture_backward(
+        *this, swap, grads, {&rows_, &w_, &b_, &mean_, &rstd_}, kind, n, approximate, has_w,
+        has_b,
+        {task_should_compute_output(0), task_should_compute_output(1),
+         task_should_compute_output(2), task_should_compute_output(3)},
+        [&] {
+          variable_list saved{rows_.unpack(shared_from_this())};
+          if (has_w) saved.push_back(w_.unpack());
+          if (has_b) saved.push_back(b_.unpack());
+          saved.push_back(rstd_.unpack());
+          if (kind != kRmsNorm && kind != kAddRmsNorm) saved.push_back(mean_.unpack());
+          return saved;
+        });
   }
   std::string name() const override { return "FusedNormBackward"; }
   void release_variables() override {

@@ -147,3 +147,27 @@ def test_quantized_forwards_pass_gradients_through_h():
         q2, s2, h2 = fops.add_rms_norm_mxfp8(x, r, 64, w)
     assert torch.equal(q.view(torch.uint8), q2.view(torch.uint8)) and torch.equal(h, h2)
     assert torch.equal(s.view(torch.uint8), s2.view(torch.uint8)) and not h2.requires_grad
+
+
+@pytest.mark.parametrize("kind,lead,shape", [(k, (5, 3), (4, 33)) for k in KINDS]
+                         + [("ln", (5, 3), (132,)), ("rms", (15,), (132,)),
+                            ("add_rms", (15,), (132,)), ("gelu_tanh", (132,), (132,))])
+@pytest.mark.parametrize("affine", [True, False])
+@pytest.mark.parametrize("backend", ["eager", "aot_eager"])
+def test_backward_under_compiled_autograd(kind, lead, shape, affine, backend):
+    """A forward in eager code whose backward compiled autograd captures: the eager gradients."""
+    from torch._dynamo import compiled_autograd
+    torch._dynamo.reset()
+    for use in ((True, True), (True, False), (False, True))[:3 if kind.startswith("add") else 1]:
+        x, r, w, b = _inputs(kind, torch.float32, lead, shape, affine)
+        _, want = _step(kind, x, r, shape, w, b, use)
+        out = _call(kind, x, r, shape, w, b)
+        g = torch.Generator().manual_seed(11)
+        ups = [torch.randn(*o.shape, generator=g).to(o) for o in out]
+        loss = sum((o * u).sum() for o, u, k in zip(out, ups, use) if k)
+        with compiled_autograd._enable(torch.compile(backend=backend, fullgraph=True)):
+            loss.backward()
+        for t, c in zip([t for t in (x, r, w, b) if t is not None], want):
+            # (a gradient that reaches nothing is zeros in one and absent in the other)
+            got = torch.zeros_like(t) if t.grad is None else t.grad
+            assert torch.equal(got, torch.zeros_like(t) if c is None else c)
