@@ -1467,12 +1467,19 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   }
   if (!g.reg_path) threads = 1024;
   if (threads < kWave * g.wpr) threads = kWave * g.wpr;
-  if (g.reg_path) threads = threads / (kWave * g.wpr) * (kWave * g.wpr);  // whole row groups
+  if (g.reg_path) {  // whole row groups
+    const int group = kWave * g.wpr;
+    threads = threads / group * group;
+    // A forced size may leave fewer threads than the GELU kernels' LDS table has entries.
+    if (gelu && threads < kGeluTabN) threads = (kGeluTabN + group - 1) / group * group;
+  }
   g.threads = threads;
   g.rgs = g.reg_path ? threads / (kWave * g.wpr) : 1;
   if (few_rows || tun.bwd_threads > 0) per_cu = 1024 / threads;  // 16 waves per CU in total
   if (tun.bwd_grid_mult >= 1 && tun.bwd_grid_mult <= 4) per_cu = tun.bwd_grid_mult;
-  const int64_t max_blocks = static_cast<int64_t>(device_cu_count()) * per_cu;
+  int64_t max_blocks = static_cast<int64_t>(device_cu_count()) * per_cu;
+  // (Five 192-thread blocks would fit a CU's 1024 threads; the workspace holds four's partial rows.)
+  if (max_blocks > workspace_partial_rows(rows)) max_blocks = workspace_partial_rows(rows);
   int64_t blocks = (rows + g.rgs - 1) / g.rgs;
   if (blocks > max_blocks) blocks = max_blocks;
   if (blocks < 1) blocks = 1;

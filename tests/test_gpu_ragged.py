@@ -106,6 +106,21 @@ def test_ragged_in_place(lib, dtype, rows, cols):
         assert (a.float() - c.float()).abs().max() <= (ulp if a.dtype == dtype else 1e-5) * scale
 
 
+@pytest.mark.parametrize("threads", ["256", "512", "1024"])
+@pytest.mark.parametrize("kind,dtype,cols", [("ln", torch.bfloat16, 1401), ("rms", torch.float16, 1030),
+                                             ("gelu_tanh", torch.bfloat16, 1401),
+                                             ("gelu_none", torch.float32, 1403),
+                                             ("ln", torch.float32, 1403)])
+def test_forced_blocks_hold_whole_row_groups(lib, monkeypatch, kind, dtype, cols, threads):
+    """Ragged rows of three waves in forced block sizes: 256 threads are one row group of 192, fewer
+    than the GELU' table has entries and so many blocks per CU that the partial rows of all of them
+    would pass the workspace."""
+    monkeypatch.setenv("FLN_BWD_THREADS", threads)
+    monkeypatch.setenv("FLN_BWD_WPR", "3")
+    capi.reload_tuning()
+    checks.test_random_shapes_against_the_oracle(lib, kind, dtype, 1500, cols, False)
+
+
 def test_streamed_grids_do_not_depend_on_the_calls_before(lib, monkeypatch, capfd):
     """The grid of a streamed forward is what its own kernel's occupancy gives, whichever flavour ran
     first: a ragged bf16 LayerNorm fits a CU twice, residual + LayerNorm (over 64 VGPRs) once."""
