@@ -562,7 +562,8 @@ enum NormKind { kLayerNorm = 0, kRmsNorm = 1, kLayerNormGelu = 2, kAddLayerNorm 
 
 // Whether a call on these tensors may pass the dispatcher by: ordinary GPU tensors, nothing that
 // watches or rewrites operator calls (dispatch modes, tracing, functorch transforms, subclasses),
-// no forward-mode tangents.
+// no forward-mode tangents, no values that the operators' dispatch would first have to write out
+// (conjugate and negative views; zero tensors, whose null pointer would pass for an absent weight).
 bool plain_call(std::initializer_list<const Tensor*> tensors) {
   if (c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing() ||
       c10::impl::tls_local_dispatch_key_set().included_.has(
@@ -572,7 +573,8 @@ bool plain_call(std::initializer_list<const Tensor*> tensors) {
                                          c10::DispatchKey::FuncTorchGradWrapper,
                                          c10::DispatchKey::FuncTorchBatched,
                                          c10::DispatchKey::Batched, c10::DispatchKey::Conjugate,
-                                         c10::DispatchKey::Negative});
+                                         c10::DispatchKey::Negative,
+                                         c10::DispatchKey::ZeroTensor});
   for (const Tensor* t : tensors) {
     if (t == nullptr || !t->defined()) continue;
     if (!t->is_cuda() || t->layout() != at::kStrided || t->key_set().has_any(special) ||

@@ -171,3 +171,17 @@ def test_backward_under_compiled_autograd(kind, lead, shape, affine, backend):
             # (a gradient that reaches nothing is zeros in one and absent in the other)
             got = torch.zeros_like(t) if t.grad is None else t.grad
             assert torch.equal(got, torch.zeros_like(t) if c is None else c)
+
+
+def test_zero_tensors_stay_refused():
+    """torch's tensors of zeros without storage: the operators refuse what their dispatch makes of
+    them (an expanded zero); a null gamma would be taken for an absent one."""
+    x = torch.randn(6, 64, device=DEV)
+    zero, big = (torch._efficientzerotensor(s, device=DEV) for s in ((64,), (6, 64)))
+    y = fops.layer_norm_gelu(x.clone().requires_grad_(), 64)
+    for call in (lambda: fops.add_rms_norm(x, x, 64, zero),
+                 lambda: fops.layer_norm_gelu(x, 64, zero, zero),
+                 lambda: fops.rms_norm_fp8(x, 64, zero), lambda: fops.add_layer_norm(x, big, 64),
+                 lambda: y.backward(big)):
+        with pytest.raises(RuntimeError, match="must be contiguous"):
+            call()
