@@ -144,3 +144,18 @@ def test_streamed_grids_do_not_depend_on_the_calls_before(lib, monkeypatch, capf
             torch.cuda.synchronize()
             grids.append(int(capfd.readouterr().err.split("fln wide: blocks=")[1].split()[0]))
     assert grids == [cus, 2 * cus] * 2
+
+
+def test_mean_sums_each_vector_by_itself(lib):
+    """fp32 rows of 4093 columns: 4 waves of 4 vectors per lane, columns 0-3, 1024-1027, ... in lane
+    0.  2^24 and then 15 ones there: three of them are lost against 2^24 in its own vector (ties
+    to even), the others arrive as sums of four; in one chain all 15 are lost."""
+    rows, cols = 3, 4093
+    x = torch.zeros(rows, cols, dtype=torch.float64)
+    for k in range(4):
+        x[:, 1024 * k:1024 * k + 4] = 1
+    x[:, 0] = 2.0 ** 24
+    want = x.sum(1)
+    _, mean, _ = ln_forward(lib, cuda(x.float()), None, None, 1e-5)
+    # sum / cols is rounded to within an ulp: 2^-23 of it
+    assert ((mean.double().cpu() * cols - want).abs() <= 3 + 2.0 ** -23 * want).all()
