@@ -75,13 +75,30 @@ def test_ragged_outputs_stay_inside(lib, dtype, rows, cols):
             assert torch.equal(out.view(rows, cols), want)
 
 
+# In place, the elements that a row's last vector shares with the one before it matter where the two
+# lie in different waves, blocks or steps: within a wave all loads come before any store.
+IN_PLACE = [(3, 600), (300, 1023), (7, 8193), (5, 20001), (300, 33001),
+            (5, 20481), (40, 20481), (300, 20481),  # starts a wave and a column block
+            (5, 32769), (40, 32769)]                # ... and a step of the streamed forward
+
+
+def test_in_place_widths_part_the_shared_elements():
+    """The widths above do what they are there for (in each element size; the quarter vectors of the
+    few-row column pass are 2 16-bit elements, or one fp32 one, which share nothing)."""
+    for cols, step in ((20481, 64), (32769, 4096)):
+        for vec in (2, 4, 8):
+            last = -(-cols // vec) - 1  # index of the last vector
+            assert (last + 1) * vec - cols == vec - 1  # one element of its own
+            assert last % 256 == 0 and (vec == 2 or last % step == 0)
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
-@pytest.mark.parametrize("rows,cols", [(3, 600), (300, 1023), (7, 8193), (5, 20001), (300, 33001)])
-def test_ragged_in_place(lib, dtype, rows, cols):
-    """y over x and dx over dy: the outputs of separate buffers, bit for bit, also where the row's
-    last vector shares elements with the one before it."""
+@pytest.mark.parametrize("rows,cols", IN_PLACE)
+def test_ragged_in_place(lib, monkeypatch, dtype, rows, cols):
+    """y over x and dx over dy, x or dres, on the routes of separate buffers (without the one-launch
+    backward, which takes no such call): the outputs of separate buffers bit for bit."""
     gen = torch.Generator().manual_seed(cols + 1)
-    x, dy = (cuda(torch.randn(rows, cols, generator=gen).to(dtype)) for _ in range(2))
+    x, dy, r = (cuda(torch.randn(rows, cols, generator=gen).to(dtype)) for _ in range(3))
     g, b = (cuda(torch.randn(cols, generator=gen).to(dtype)) for _ in range(2))
     p = capi.ptr
     code, st = capi.dtype_code(x), capi.stream()
@@ -91,17 +108,27 @@ def test_ragged_in_place(lib, dtype, rows, cols):
                                          1e-5, st))
     assert torch.equal(y, y0)
     ws, nb = workspace(lib, rows, cols, x)
-    outs = []
-    for inplace in (False, True):
-        d = dy.clone()
-        dx = d if inplace else torch.empty_like(d)
+
+    def backward(dres, over):
+        t = {"dy": dy.clone(), "x": x.clone(), "dres": r.clone() if dres else None}
+        dx = t[over] if over else torch.empty_like(x)
         dg, db = torch.empty(cols, device="cuda"), torch.empty(cols, device="cuda")
-        capi.check(lib.fln_layernorm_backward(p(d), p(x), p(mean), p(rstd), p(g), None, p(dx),
-                                              p(dg), p(db), rows, cols, code, capi.F32, p(ws), nb,
-                                              st))
-        outs.append((dx, dg, db))
+        capi.check(lib.fln_layernorm_backward(p(t["dy"]), p(t["x"]), p(mean), p(rstd), p(g),
+                                              p(t["dres"]), p(dx), p(dg), p(db), rows, cols, code,
+                                              capi.F32, p(ws), nb, st))
+        return dx, dg, db
+
+    small = backward(False, None)  # by whatever route
+    monkeypatch.setenv("FLN_BWD_SMALL_ROWS", "-1")
+    capi.reload_tuning()
+    for dres in (False, True):
+        want = backward(dres, None)
+        for over in ("dy", "x", "dres")[:3 if dres else 2]:
+            for a, c in zip(backward(dres, over), want):
+                assert torch.equal(a, c), (dres, over)
+    # The one launch sums in another order: within a rounding of the largest value.
     ulp = {torch.float32: 2.0 ** -20, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
-    for a, c in zip(*outs):  # another route may sum in another order: one rounding of the type
+    for a, c in zip(small, backward(False, None)):
         scale = c.float().abs().max()
         assert (a.float() - c.float()).abs().max() <= (ulp if a.dtype == dtype else 1e-5) * scale
 

@@ -37,8 +37,24 @@ def _cases():
 
 @pytest.mark.parametrize("kind,dtype,rows,cols,shifted", list(_cases()),
                          ids=lambda v: str(v)[6:] if isinstance(v, torch.dtype) else str(v))
-def test_small_backward(lib, kind, dtype, rows, cols, shifted):
+def test_small_backward(lib, monkeypatch, capfd, kind, dtype, rows, cols, shifted):
+    monkeypatch.setenv("FLN_DEBUG_GEOMETRY", "1")
+    capi.reload_tuning()
+    capfd.readouterr()
     checks.test_random_shapes_against_the_oracle(lib, kind, dtype, rows, cols, shifted)
+    err = capfd.readouterr().err
+    assert err.count("fln backward:") == 1, err
+    # 16 waves of 8 vectors per lane at most; of those few rows and 16-bit GELU take the two passes,
+    # and 16-bit GELU of 4 vectors per lane too unless every block has a CU of its own.
+    vec = 4 if dtype == torch.float32 else 8
+    nvec, cus = -(-cols // vec), torch.cuda.get_device_properties(0).multi_processor_count
+    gelu16 = kind.startswith("gelu") and vec == 8
+    small = cols >= vec and nvec <= 8192 and rows <= cus
+    if nvec > 4096:
+        small = small and not gelu16 and rows >= (32 if vec == 8 and cols % vec else 16)
+    elif nvec > 2048 and gelu16:
+        small = small and rows + -(-nvec // 64) <= cus
+    assert ("-> small" in err) == small, err
 
 
 # Around the rows and widths at which the two passes take over from the one launch, and those of
