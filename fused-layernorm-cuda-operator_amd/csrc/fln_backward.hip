@@ -729,10 +729,14 @@ __global__ __launch_bounds__(NT) void bwd_lds_kernel(const BwdParams p) {
 // 5 streams (x, dy twice, dx once) instead of 3, but every access is a coalesced vector stream
 // and no thread holds more than eight vectors per array.  The row statistics read x and dy with
 // the default cache policy, so that the column pass, which reads them for the last time and
-// streams, finds in the 256 MB memory-side cache what fits there (backward calls, us, streaming
+// streams, finds part of them in the 256 MB memory-side cache (backward calls, us, streaming
 // loads in the first pass / default there / default in both: fp32 256 x 65536 60.8 / 58.4 / 61.9,
 // 1000 x 20001 87.4 / 79.8 / 80.4; bf16 300 x 100000 84.3 / 78.5 / 78.4, 2048 x 40000 164.5 /
-// 155.2 / 168.4, 8192 x 40000 632 / 618 / -, 64 x 1048576 114.0 / 115.3 / 119.0).  The column
+// 155.2 / 168.4, 8192 x 40000 632 / 618 / -, 256 x 1048576 468 / 451 / -).  A few sizes lose among
+// neighbours that gain, and no line by size parts them: bf16 64 x 1048576 114.0 / 115.3 / 119.0
+// (64 x 917504 117.0 / 105.0, 128 x 1048576 228 / 224), 64 x 1040000 124.5 / 128.2 (64 x 1060000
+// 137.3 / 130.4), 512 x 131072 119.0 / 122.0 (512 x 135168 138.9 / 134.4, 1024 x 65536 121.1 /
+// 117.7), fp32 300 x 131072 140.4 / 145.0 (240 x 131072 108.5 / 104.1).  The column
 // pass taking the rows from the last one on, so as to start on those read last, measured no
 // better than in order (155.2 -> 154.8, 618 -> 626, fp32 4096 x 20480 296 -> 303).
 constexpr int kWideThreads = 256;
@@ -1368,8 +1372,8 @@ BwdGeometry backward_geometry(int64_t rows, int64_t cols, int dtype, bool vec_ok
   // backward calls, us, 4 -> 8 elements per lane: 300 x 768 9.31 -> 8.81, 4096 x 768 13.79 ->
   // 13.19, 16384 x 768 31.46 -> 30.26, 16384 x 1024 38.12 -> 37.68, 8192 x 2048 38.60 ->
   // 38.13, 4096 x 3072 32.62 -> 31.06, 1024 x 4096 17.74 -> 17.14, 8192 x 4096 70.54 -> 69.36
-  // (RMSNorm 69.02 -> 67.77); 32 x 768 and 1024 x 1024 tied.  The fp32 scalar path (rows not
-  // whole 16-byte vectors) keeps 4.
+  // (RMSNorm 69.02 -> 67.77); 32 x 768 and 1024 x 1024 tied.  The fp32 scalar path (rows of at
+  // most kScalarCols columns off the vectors' alignment) keeps 4.
   const Tuning& tun = tuning();
   const int epl = tun.bwd_epl > 0 ? tun.bwd_epl : (es == 4 && g.vec == 1 ? 4 : 8);
   int cap = (epl >= g.vec ? epl : g.vec) / g.vec;
@@ -1657,9 +1661,10 @@ int launch_backward(const BwdParams& p0, int dtype, void* dgamma, void* dbeta, i
   // gradient is requested, then the row statistics of the two-pass path [rows, splits, 2]
   // (16-byte aligned: ld is a multiple of 4).  At most fln_backward_workspace_bytes() (blocks <=
   // workspace_partial_rows on every path; splits within what that bound leaves).
-  // A column pass with one block row (columns >= 2 x CUs column tiles, or at most 8 rows) holds the
-  // final column sums: it writes dgamma / dbeta itself, without partial rows or the column
-  // reduction (the same bits: the reduction of one partial row only converts it).
+  // A column pass with one block row (column tiles enough for the device, or so few rows that one
+  // block row takes them: at most 8, of fp32 16) holds the final column sums: it writes dgamma /
+  // dbeta itself, without partial rows or the column reduction (the same bits: the reduction of one
+  // partial row only converts it).
   const bool direct = geo.two_pass && geo.blocks == 1;
   const int64_t part = (dgamma || dbeta) && !direct ? 2 * geo.blocks * ld : 0;
   // Row statistics of the two-pass path: fewer rows than the statistics pass has blocks split

@@ -13,12 +13,16 @@
 //     of a column are added through LDS.
 // Both roles take unaligned vectors (RaggedRow), so any width of at least one vector runs here.
 //
-// Taken for at most one row per CU.  Backward calls, us, before -> here: fp32 32 x 768 6.4 -> 3.6, 128
+// Taken for at most one row per CU, where no width that it takes loses.  Backward calls, us, before -> here: fp32 32 x 768 6.4 -> 3.6, 128
 // x 768 6.9 -> 3.8, 256 x 768 7.7 -> 4.7, 256 x 16384 27.4 -> 18.2, 256 x 32768 36.8 -> 36.5; bf16 64 x
 // 4096 8.1 -> 4.3, 256 x 1024 8.4 -> 4.8, 256 x 8192 19.5 -> 8.1, 200 x 12288 19.9 -> 7.6, 100 x 40000
 // 25.3 -> 14.7, 1 x 32768 11.5 -> 6.7; erf GELU 64 x 4096 9.5 -> 8.0, 100 x 30000
 // 32.3 -> 15.2; residual gradient 200 x 50000 41.1 -> 28.2.  More rows amortize the two stages'
-// overhead and read x and dy once.  What bounds it: one launch and two dependent round trips to memory
+// overhead and read x and dy once: wide ones soon (us, two stages / here: bf16 512 x 4097 15.5 / 13.8,
+// 768 x 4097 17.7 / 18.8; fp32 768 x 2048 10.8 / 9.7, 1000 x 2048 11.2 / 12.0), narrow ones only past
+// 1000 (fp32 512 x 768 7.8 / 6.2, 1000 x 768 10.8 / 8.7, 1500 x 768 9.6 / 11.9; bf16 1000 x 4096 14.8 /
+// 13.7, 1500 x 4096 16.4 / 19.1), so that a limit by rows and columns would serve more calls.  What
+// bounds it: one launch and two dependent round trips to memory
 // for narrow rows; the bandwidth of the few CUs that hold a row for wide ones.
 #include <type_traits>
 
@@ -319,9 +323,10 @@ bool backward_is_small(const BwdParams& p, const void* dgamma, const void* dbeta
   if (p.rows > limit || p.rows * p.cols * es >= int64_t(1) << 31) return false;
   // The widest rows (8 vectors per lane) are bound by the one CU that holds a row: with a few rows
   // the two passes spread each over many CUs (backward calls, us, here / two passes: bf16 LN 4 x
-  // 50000 11.8 / 8.4, 16 x 50000 12.2 / 12.0, 30 x 50000 12.6 / 15.0, off the 16-byte grid 4 x 60001
-  // 15.4 / 9.4, 16 x 60001 15.8 / 13.2, 30 x 60001 16.2 / 15.6; fp32 4 x 32768 8.5 / 7.2, 16 x 20001
-  // 8.2 / 10.4, 16 x 32768 8.8 / 10.6).
+  // 50000 11.8 / 8.4, 16 x 50000 12.6 / 11.6, 20 x 50000 12.8 / 12.8, 40 x 50000 13.6 / 15.8; widths
+  // that are no whole vectors 4 x 60001 15.4 / 9.4, 16 x 60001 15.8 / 13.2, 32 x 60001 16.8 / 15.5, 40
+  // x 60001 17.2 / 16.9; fp32 4 x 32768 8.5 / 7.2, 16 x 20001 8.2 / 10.3, 16 x 32768 9.4 / 9.9).  The
+  // rule looks at the width, not at the pointers.
   // So are 16-bit rows with GELU, whose derivative is taken twice per element: 8 vectors per lane
   // never (64 x 50000 24.5 / 21.2, 128 x 50000 28.3 / 28), 4 only while every block has its own CU
   // (200 x 20000 23.1 / 31.6, but 256 x 20000 35.4 / 34.2, 256 x 32768 38.1 / 33.1).

@@ -13,8 +13,9 @@
 //   * optional GELU epilogue (erf or tanh),
 //   * optional residual add (h = x + r rounded to the I/O type, statistics over h),
 //   * output in the I/O type, or OCP fp8 e4m3fn codes plus a per-row fp32 scale.
-// Rows too long for registers (or odd rows beyond 4096 elements) take a looped fallback that
-// keeps the same arithmetic but re-reads the row (from L2) on each pass.
+// Rows too long for registers are parked in LDS, split over several blocks (few rows) or streamed in
+// passes; fp64 and rows of 2 GiB or more take a looped kernel that keeps the same arithmetic but
+// re-reads the row on each pass.
 //
 // The kernels live in fln_forward_impl.h and are instantiated per I/O type in
 // fln_forward_{f32,bf16,f16,f64}.hip; this file validates arguments and holds the entry points.

@@ -65,7 +65,7 @@ __device__ __forceinline__ float row_allreduce(float v, float* slot, int wpr, in
 // A 16-byte copy at 2-byte alignment moves 5.0-5.4 TB/s here against 5.9 aligned; the scalar path
 // this replaced (one element per lane and load, 128 bytes per wave and instruction) was bound by
 // its load and store issue at 2.2 TB/s.  Forward, us, scalar -> ragged:
-//   LayerNorm bf16 8192 x 4098 50.6 -> 28.2, 8192 x 4095 35.3 -> 27.0, 4000 x 4097 28.8 -> 18.9,
+//   LayerNorm bf16 8192 x 4098 50.6 -> 28.2, 8192 x 4095 35.3 -> 26.7, 4000 x 4097 28.8 -> 18.5,
 //   4000 x 9999 55.1 -> 35.2, 16384 x 1023 18.2 -> 14.9; fp32 5000 x 5003 43.4 -> 39.9; residual +
 //   LayerNorm bf16 8000 x 2050 43.9 -> 26.2; LN + GELU erf bf16 14591 x 1146 34.9 -> 22.5, tanh
 //   fp16 6001 x 1023 12.0 -> 10.0; LN -> fp8 bf16 9000 x 3001 41.3 -> 23.7; LN -> MXFP8 bf16 4096
@@ -1351,8 +1351,8 @@ int launch_reg_vpl(const FwdParams& p, int vpl, int fit, int threads, hipStream_
     switch (vpl) {
       case 2: return launch_reg_fit<T, FP8, RES, GELU, VEC, 2>(p, fit, threads, s);
       case 4: return launch_reg_fit<T, FP8, RES, GELU, VEC, 4>(p, fit, threads, s);
-      // Odd and six-vector tiles (3, 5, 6, 7 vectors per lane): exact tilings only, in blocks of
-      // at most 256 threads, for the 16-bit flavours that the plan gives them.
+      // Odd and six-vector tiles (3, 5, 6, 7 vectors per lane): exact tilings, in blocks of at most
+      // 256 threads, for the 16-bit flavours that the plan gives them; ragged rows 3 and 5.
       case 3: return launch_reg_odd<T, FP8, RES, GELU, VEC, 3>(p, fit, threads, s);
       case 5: return launch_reg_odd<T, FP8, RES, GELU, VEC, 5>(p, fit, threads, s);
       case 6: return launch_reg_odd<T, FP8, RES, GELU, VEC, 6>(p, fit, threads, s);
@@ -1967,11 +1967,15 @@ inline FwdGeometry fwd_geometry(int64_t rows, int64_t nvec, int cap, int wide_ca
 
 // The tiling of ragged rows, whose width is as a rule no whole tile: the fewest waves per row whose
 // tile holds at most 1/8 more vectors than the tightest one.  Masked slots cost issue slots, and
-// extra waves cross-wave reductions (LayerNorm, us, waves x vectors per lane): bf16 4000 x 4097
-// (513 vectors) 2 x 5 15.9, 3 x 3 16.6, 9 x 1 17.4, 4 x 4 20.3; 6000 x 6001 3 x 4 31.8, 12 x 1
-// 31.5, 2 x 8 does not fit; 4000 x 9999 10 x 2 35.1, 4 x 5 37.8, 16 x 2 42.2; fp32 3000 x 3003
-// 3 x 4 15.6, 2 x 8 16.8; 5000 x 5003 5 x 4 38.2, 4 x 8 41.4; residual + LayerNorm bf16 8000 x
-// 2050 1 x 5 26.0, 2 x 4 28.5.  Vectors per lane: of 16-bit rows up to 4 in one to four waves (5 in
+// extra waves cross-wave reductions.  LayerNorm calls with statistics, us, waves x vectors per lane
+// (the rule's first), inputs and outputs rotating over 900 MB: bf16 16384 x 1023 1 x 2 15.0, 2 x 1
+// 15.6; 9000 x 2049 1 x 5 18.2, 2 x 3 18.8, 3 x 2 19.9, 5 x 1 20.9; 8192 x 4095 2 x 4 26.6, 3 x 3
+// 29.6, 8 x 1 29.9; 4000 x 4097 (513 vectors) 2 x 5 18.4, 3 x 3 16.5, 9 x 1 17.7, 5 x 2 17.8; 8192
+// x 4098 2 x 5 28.6, 3 x 3 27.6, 9 x 1 29.0; 6000 x 6001 3 x 4 33.7, 12 x 1 31.5, 4 x 3 32.8; 4000 x
+// 9999 10 x 2 35.1, 16 x 2 42.2; fp32 3000 x 3003 3 x 4 16.2, 6 x 2 15.9, 12 x 1 16.0; 5000 x 5003
+// 5 x 4 39.9, 10 x 2 38.3; residual + LayerNorm bf16 8000 x 2050 1 x 5 26.2, 3 x 2 27.4, 2 x 3 28.3.
+// So the rule's tile is the fastest of bf16 rows up to 4096 columns and of 9999, and elsewhere 2 to
+// 11% slower than the best one.  Vectors per lane: of 16-bit rows up to 4 in one to four waves (5 in
 // one or two) and up to 2 in more; of fp32 rows 1, 2 or 4 (16 waves x 4: 16384 columns, the 16-bit
 // limit 16 x 2).  Longer rows take the streamed kernel.
 inline FwdGeometry ragged_geometry(int64_t rows, int64_t nvec, int vec, bool erf, int forced_wpr,

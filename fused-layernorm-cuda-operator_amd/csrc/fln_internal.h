@@ -164,7 +164,7 @@ struct BwdGeometry {
   int vec;        // elements per vector access
   int col_vec;    // two-pass: elements per access of the column pass
   bool ragged;    // rows off the 16-byte grid: unaligned vectors
-  int vpl;        // vectors per lane (power of two, <= 16)
+  int vpl;        // vectors per lane (1 to 4; 0 off the register path)
   int wpr;        // waves per row
   int threads;    // block size
   int rgs;        // row groups per block

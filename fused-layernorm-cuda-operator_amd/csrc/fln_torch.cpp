@@ -896,7 +896,9 @@ Tensor rms_norm_autograd(const Tensor& input, int64_t normalized, const OptT& we
 // gradients for the statistics outputs (a training step of 8 x 768 rows, host-bound, us:
 // layer_norm_gelu 155, add_rms_norm 148, FusedLayerNorm over [64, 32, 32] 143; nn.LayerNorm 73).
 // Here one node holds what the operators' formulas save (the normalized rows, weight, bias, mean,
-// rstd) and its backward calls the same functions, so outputs and gradients are the same bits.
+// rstd) and its backward calls the same functions.  Outputs are the same bits, and gradients too but
+// where a residual sum is not used any further: the operators add a gradient of zeros then, in the
+// kernel's residual form, and round once more (at most an ulp of a 16-bit dx apart).
 // ------------------------------------------------------------------------------------------
 
 struct FusedNormBackward : public torch::autograd::Node {

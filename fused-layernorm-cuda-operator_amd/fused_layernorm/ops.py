@@ -295,9 +295,10 @@ def _flat_param(p: Optional[torch.Tensor]):
     return None if p is None else p.reshape(-1)
 
 
-# The eager paths below pass the operators by where nothing can tell the difference: ordinary
-# tensors outside torch.compile, with no __torch_function__ mode; the extension refuses the rest
-# (dispatch modes, tracing, functorch transforms, forward-mode tangents).
+# The eager paths below pass the operators by where nothing looks on: ordinary tensors outside
+# torch.compile, with no __torch_function__ mode; the extension refuses the rest (dispatch modes,
+# tracing, functorch transforms, forward-mode tangents, zero tensors).  Their autograd nodes take the
+# operators for a backward that something watches, compiled autograd's capture among them.
 _ORDINARY = (torch.Tensor, torch.nn.Parameter)
 _compiling = torch.compiler.is_compiling
 _function_modes = torch._C._len_torch_function_stack

@@ -74,7 +74,8 @@ int fln_layernorm_forward(const void* x, const void* gamma, const void* beta, vo
 
 /* Workspace (bytes) the backward entry points use: the two-stage column reduction's partial
  * rows and, for rows wider than the register and LDS kernels hold (16-bit or fp32 rows of more
- * than 16384 columns, long rows on the unaligned path), per-row statistics.  Required whenever
+ * than 16384 columns; fp32 rows off the 16-byte grid of more than 8192), per-row statistics.
+ * Required whenever
  * dgamma / dbeta is requested; passing it for dx alone lets such rows take the two-pass
  * kernels instead of the slower looped one. */
 size_t fln_backward_workspace_bytes(int64_t rows, int64_t cols, int dtype);
@@ -248,10 +249,10 @@ const char* fln_version(void);
 int fln_hip_version(void);
 const char* fln_error_string(int code);
 /* Re-reads the FLN_* tuning and debugging environment variables (FLN_FORCE_LOOP, FLN_FWD_EPL,
- * FLN_FWD_WPR, FLN_FWD_GRID_MULT, FLN_FWD_NO_LDS, FLN_FWD_NO_WIDE, FLN_DEBUG_GEOMETRY,
- * FLN_BWD_EPL, FLN_BWD_WPR, FLN_BWD_THREADS, FLN_BWD_NO_LDS, FLN_BWD_NO_TWO_PASS,
- * FLN_BWD_SMALL_ROWS); they are
- * otherwise read once, at the first launch.  No counterpart in the reference: for tests and
+ * FLN_FWD_WPR, FLN_FWD_GRID_MULT, FLN_FWD_NO_LDS, FLN_FWD_NO_WIDE, FLN_FWD_NO_SPLIT,
+ * FLN_FWD_SPLITS, FLN_FWD_SPLIT_ROWS, FLN_DEBUG_GEOMETRY, FLN_BWD_EPL, FLN_BWD_WPR,
+ * FLN_BWD_THREADS, FLN_BWD_GRID_MULT, FLN_BWD_NO_LDS, FLN_BWD_NO_TWO_PASS, FLN_BWD_STAT_SPLITS,
+ * FLN_BWD_COLPASS_PER_CU, FLN_BWD_SMALL_ROWS); they are otherwise read once, at the first launch.  No counterpart in the reference: for tests and
  * tuning sweeps. */
 void fln_reload_tuning(void);
 

@@ -1,5 +1,6 @@
 """The eager differentiable paths that pass the operators by: the operators' outputs and gradients
-bit for bit, and the operators themselves wherever something watches the call."""
+(bit for bit but where a residual sum is not used), and the operators themselves wherever something
+watches the call."""
 from __future__ import annotations
 
 import pytest
