@@ -219,7 +219,8 @@ int fln_fp8_e4m3fn_encode(const float* x, uint8_t* q, int64_t n, void* stream);
 
 typedef struct fln_forward_plan {
   int route;            /* FLN_ROUTE_* */
-  int vector_elems;     /* elements per lane load: 16 bytes' worth on the vector path, else 1 */
+  int vector_elems;     /* elements per lane load: 16 bytes' worth (also off the 16-byte grid, from
+                         * 257 columns on), else 1 */
   int waves_per_row;    /* register route: wave64s per row (0 on the other routes) */
   int vectors_per_lane; /* register route: vectors of the row per lane (0 on the other routes) */
   int exact;            /* register route: 1 if no lane holds a masked slot */
